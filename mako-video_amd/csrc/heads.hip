@@ -16,7 +16,7 @@
 //   (the norm factor is the group's).
 // - The workgroup stages the two norm weight vectors and its rows' cos / sin tables in LDS once.
 // - A padding slot of the cube map writes zeros and reads nothing.
-// mh3_heads_partial_pool adds cube_pool to the same pass (heads_pool_kernel, a workgroup per cube): the selector's
+// mh3_heads_partial_pool adds cube_pool to the same pass (heads_pool_kernel, workgroups of one cube each): the selector's
 // cube means come from the values as they are stored, so q and k are not read back from HBM.
 #include "mh3_common.hpp"
 
@@ -41,8 +41,7 @@ struct HeadsParams {
     uint16_t* out[3];
     uint64_t qkv_stride, ohs, ors;
     uint32_t rows, model_rows, heads, half, per_row, rows_per_block;
-    uint32_t row_begin; // first output row of the launch; it covers rows row_begin .. rows - 1
-    FastDiv div_row, div_heads;
+    FastDiv div_row, div_heads, div_half;
     float eps;
 };
 
@@ -125,14 +124,12 @@ __device__ __forceinline__ void stage_weights(float* wt, const float* qw, const 
     }
 }
 
-__global__ __launch_bounds__(kHeadsThreads) void heads_kernel(HeadsParams p)
+// Output rows r0 .. r0 + nr - 1 (nr <= rows_per_block) by a workgroup of kHeadsThreads. LDS: the norm weights w [2][128]
+// (q, then k); the rows' model rows src [rows_per_block] (-1: padding); their cos and sin tables [rows_per_block][half]
+// each.
+__device__ __forceinline__ void heads_rows(const HeadsParams& p, uint32_t r0, uint32_t nr, float* lds)
 {
-    // LDS: the norm weights w [2][128] (q, then k); the rows' model rows src [rows_per_block] (-1: padding); their
-    // cos and sin tables [rows_per_block][half] each.
-    extern __shared__ float lds[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, part = lane & 15u, group = tid >> 4;
-    const uint32_t r0 = p.row_begin + blockIdx.x * p.rows_per_block;
-    const uint32_t nr = min(p.rows_per_block, p.rows - r0);
     float* wt = lds;
     int32_t* srcs = reinterpret_cast<int32_t*>(lds + 256);
     float* ct = lds + 256 + ((p.rows_per_block + 3u) & ~3u); // 16-byte aligned
@@ -188,15 +185,26 @@ __global__ __launch_bounds__(kHeadsThreads) void heads_kernel(HeadsParams p)
     }
 }
 
-// heads_partial fused with cube_pool over its output: a workgroup per cube (512 threads). Output rows row0 + 64 c + l
-// (slot l = 4 s + dx, s = dt * 4 + dy) are produced as heads_kernel produces them, and the cube's q and k means are
-// summed from the rounded values as they are stored, in cube_pool_kernel's order: for each dx, slots s = 0 .. 15 in
-// turn from zero (a slot outside the grid adds zero), then (dx 0 + dx 1) + (dx 2 + dx 3), divided by the token count.
-// The outputs are therefore bit-identical to heads_partial followed by cube_pool in the gathered layout.
-// A wave takes four consecutive head vectors of a row (one a 16-lane group), so each of its loads reads 1 KB of a
-// row; a group sums its head vector over dx 0..3 in turn, each over s = 0 .. 15, and combines the four partial sums
-// in its own registers. Taking one head vector a wave instead (the four groups the four dx, combined by lane
-// exchanges) read four 256-byte pieces of four rows a load and measured 3-4% slower.
+__global__ __launch_bounds__(kHeadsThreads) void heads_kernel(HeadsParams p)
+{
+    extern __shared__ float lds[];
+    const uint32_t r0 = blockIdx.x * p.rows_per_block;
+    heads_rows(p, r0, min(p.rows_per_block, p.rows - r0), lds);
+}
+
+// heads_partial fused with cube_pool over its output: a workgroup (512 threads) per cube and 8 consecutive head vectors
+// of its rows. Output rows row0 + 64 c + l (slot l = 4 s + dx, s = dt * 4 + dy) are produced as heads_kernel produces
+// them, and the cube's q and k means are summed from the rounded values as they are stored, in cube_pool_kernel's
+// order: for each dx, slots s = 0 .. 15 in turn from zero (a slot outside the grid adds zero), then (dx 0 + dx 1) +
+// (dx 2 + dx 3), divided by the token count. The outputs are therefore bit-identical to heads_partial followed by
+// cube_pool.
+// A wave takes four consecutive head vectors (one a 16-lane group, so a load reads 1 KB of a row) and one dx, so two
+// sets of four waves cover the workgroup's 8 vectors and the four dx sums meet in LDS. HBM-bound where the cubes fill
+// the chip; a workgroup that took a whole cube left it idle on short clips (30 cubes, 40 heads: 177 us, now 30) and
+// unevenly filled at 960 x 544 (400 cubes, 56 heads: 461 -> 417 us; 2016 cubes, 40 heads: 1.63 -> 1.53 ms). The
+// tables' loads are all issued before the first is stored (one after the other, each behind its map entry, they cost
+// 8% at 2016 cubes). Two to six workgroups a cube, each looping over its vectors, measured between the two.
+// The rows before and after the cubes' (the dense rows) go to workgroups of the same launch.
 struct HeadsPoolParams {
     HeadsParams hp;
     float* qc;
@@ -205,18 +213,28 @@ struct HeadsPoolParams {
     uint64_t row0; // gathered: output row of cube 0's slot 0; grid: the model row of grid position (0, 0, 0)
     uint32_t gt, gh, gw, cw, plane, cubes;
     uint32_t grid; // nonzero: no map, each token's row read and written at its model row (the grid layout)
+    uint32_t parts; // workgroups a cube: workgroup i of them takes the head vectors 8 i .. + 7 of its rows
+    uint32_t cube_wgs, wgs0, video0, video1; // workgroups of the cubes; then those of output rows [0, video0) (wgs0 of
+                                             // them) and [video1, rows), the rows before and after the cubes'
 };
 constexpr uint32_t kPoolThreads = 512;
-constexpr int kPoolU = 8;                           // slots a group has in flight
+constexpr int kTabU = 6;                            // table values a thread has in flight (64 x 48 in one turn)
+constexpr int kPoolU = 4;                           // slots a group has in flight (8: equal, and spills)
 
-// At most 128 registers (two workgroups a CU): left to itself the compiler takes more than that.
+// At most 128 registers (two workgroups a CU).
 __global__ __launch_bounds__(kPoolThreads) __attribute__((amdgpu_waves_per_eu(4))) void
 heads_pool_kernel(HeadsPoolParams pp)
 {
     const HeadsParams& p = pp.hp;
     extern __shared__ float lds[];
+    if (blockIdx.x >= pp.cube_wgs) {
+        const uint32_t d = blockIdx.x - pp.cube_wgs, before = d < pp.wgs0;
+        const uint32_t r0 = before ? d * p.rows_per_block : pp.video1 + (d - pp.wgs0) * p.rows_per_block;
+        heads_rows(p, r0, min(p.rows_per_block, (before ? pp.video0 : p.rows) - r0), lds);
+        return;
+    }
     const uint32_t tid = threadIdx.x, lane = tid & 63u, part = lane & 15u, grp = lane >> 4, wave = tid >> 6;
-    const uint32_t c = blockIdx.x;
+    const uint32_t c = blockIdx.x / pp.parts, part_of = blockIdx.x - c * pp.parts;
     const uint64_t orow0 = pp.row0 + uint64_t(c) * 64u;
     float* wt = lds;
     int32_t* srcs = reinterpret_cast<int32_t*>(lds + 256);
@@ -240,85 +258,90 @@ heads_pool_kernel(HeadsPoolParams pp)
     };
     if (tid < 64u)
         srcs[tid] = src_of(tid);
-    for (uint32_t i = tid; i < 64u * p.half; i += kPoolThreads) {
-        const uint32_t l = i / p.half, col = i - l * p.half;
-        const int32_t src = src_of(l);
-        ct[i] = src >= 0 ? p.cos_t[uint64_t(src) * p.half + col] : 0.0f;
-        st[i] = src >= 0 ? p.sin_t[uint64_t(src) * p.half + col] : 0.0f;
-    }
     const uint32_t nt = min(4u, pp.gt - cube_t * 4u), ny = min(4u, pp.gh - cube_y * 4u), nx = min(4u, pp.gw - cube_x * 4u);
-    if (pp.counts && tid == 0)
+    if (pp.counts && tid == 0 && part_of == 0)
         pp.counts[c] = int32_t(nt * ny * nx);
+    __syncthreads();
+    // The tables, every load of a thread in flight at once.
+    for (uint32_t i0 = tid; i0 < 64u * p.half; i0 += kPoolThreads * kTabU) {
+        float cv[kTabU], sv[kTabU];
+#pragma unroll
+        for (int u = 0; u < kTabU; ++u) {
+            const uint32_t i = i0 + kPoolThreads * uint32_t(u), l = p.div_half.div(i);
+            const int32_t src = l < 64u ? srcs[l] : -1;
+            const uint64_t at = uint64_t(src >= 0 ? src : 0) * p.half + (i - l * p.half);
+            cv[u] = src >= 0 ? p.cos_t[at] : 0.0f;
+            sv[u] = src >= 0 ? p.sin_t[at] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < kTabU; ++u) {
+            const uint32_t i = i0 + kPoolThreads * uint32_t(u);
+            if (i < 64u * p.half)
+                ct[i] = cv[u], st[i] = sv[u];
+        }
+    }
     __syncthreads();
 
     const RotLane rl = rot_lane(lane, p.half);
     const float n = float(nt * ny * nx);
-    const uint32_t blocks = (p.per_row + 3u) / 4u;
-    for (uint32_t b = wave; b < blocks; b += kPoolThreads / 64u) {
-        const uint32_t j = b * 4u + grp;
-        const bool live = j < p.per_row;
-        const uint32_t jj = live ? j : 0u;
-        const uint32_t kind = p.div_heads.div(jj), h = jj - kind * p.heads;
-        const float* wk = wt + 128u * min(kind, 1u);
-        uint16_t* const out = (kind == 0u ? p.out[0] : kind == 1u ? p.out[1] : p.out[2]) + uint64_t(h) * p.ohs;
-        float p01[8], p2[8];
+    float4* const sums = reinterpret_cast<float4*>(st + max(64u * p.half, 8u)); // [2][wave][lane]
+    const uint32_t dx = wave & 3u;
+    const uint32_t s_end = pp.grid ? 4u * nt : 16u; // the grid layout: frames of slots past its edge are no rows
+    const uint32_t j = part_of * 8u + (wave >> 2) * 4u + grp;
+    const bool live = j < p.per_row;
+    const uint32_t jj = live ? j : 0u;
+    const uint32_t kind = p.div_heads.div(jj), h = jj - kind * p.heads;
+    const float* wk = wt + 128u * min(kind, 1u);
+    uint16_t* const out = (kind == 0u ? p.out[0] : kind == 1u ? p.out[1] : p.out[2]) + uint64_t(h) * p.ohs;
+    const bool x_ok = dx < nx;
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+        acc[e] = 0.0f;
 #pragma unroll 1
-        for (uint32_t dx = 0; dx < 4u; ++dx) {
-            const bool x_ok = cube_x * 4u + dx < pp.gw;
-            float acc[8];
+    for (uint32_t s0 = 0; s0 < s_end; s0 += kPoolU) {
+        uint4 raw[kPoolU];
+        int32_t src_r[kPoolU];
 #pragma unroll
-            for (int e = 0; e < 8; ++e)
-                acc[e] = 0.0f;
-#pragma unroll 1
-            for (uint32_t s0 = 0; s0 < 16u; s0 += kPoolU) {
-                uint4 raw[kPoolU];
-                int32_t src_r[kPoolU];
+        for (int u = 0; u < kPoolU; ++u) {
+            const int32_t src = live ? srcs[(s0 + uint32_t(u)) * 4u + dx] : -1;
+            src_r[u] = src;
+            raw[u] = src >= 0 ? ld_stream(reinterpret_cast<const uint4*>(
+                                    p.qkv + uint64_t(src) * p.qkv_stride + 128u * jj + 8u * part))
+                              : uint4{0u, 0u, 0u, 0u};
+        }
 #pragma unroll
-                for (int u = 0; u < kPoolU; ++u) {
-                    const int32_t src = live ? srcs[(s0 + uint32_t(u)) * 4u + dx] : -1;
-                    src_r[u] = src;
-                    raw[u] = src >= 0 ? ld_stream(reinterpret_cast<const uint4*>(
-                                            p.qkv + uint64_t(src) * p.qkv_stride + 128u * jj + 8u * part))
-                                      : uint4{0u, 0u, 0u, 0u};
-                }
+        for (int u = 0; u < kPoolU; ++u) {
+            const uint32_t s = s0 + uint32_t(u), l = s * 4u + dx;
+            uint4 o = head_vector(raw[u], kind, wk, ct + l * p.half + rl.ci, st + l * p.half + rl.ci, rl,
+                                  part, p.eps);
+            o = src_r[u] >= 0 ? o : uint4{0u, 0u, 0u, 0u};
+            // Gathered: every slot's row is written (a padding slot's zeros); grid: a token's own row only.
+            const uint64_t orow = pp.grid ? uint64_t(src_r[u] >= 0 ? src_r[u] : 0) : orow0 + l;
+            if (live && (!pp.grid || src_r[u] >= 0))
+                st_stream(reinterpret_cast<uint4*>(out + orow * p.ors + 8u * part), o);
+            const bool ok = x_ok && cube_t * 4u + (s >> 2) < pp.gt && cube_y * 4u + (s & 3u) < pp.gh;
+            const uint32_t w[4] = {o.x, o.y, o.z, o.w};
 #pragma unroll
-                for (int u = 0; u < kPoolU; ++u) {
-                    const uint32_t s = s0 + uint32_t(u), l = s * 4u + dx;
-                    uint4 o = head_vector(raw[u], kind, wk, ct + l * p.half + rl.ci, st + l * p.half + rl.ci, rl,
-                                          part, p.eps);
-                    o = src_r[u] >= 0 ? o : uint4{0u, 0u, 0u, 0u};
-                    // Gathered: every slot's row is written (a padding slot's zeros); grid: a token's own row only.
-                    const uint64_t orow = pp.grid ? uint64_t(src_r[u] >= 0 ? src_r[u] : 0) : orow0 + l;
-                    if (live && (!pp.grid || src_r[u] >= 0))
-                        st_stream(reinterpret_cast<uint4*>(out + orow * p.ors + 8u * part), o);
-                    const bool ok = x_ok && cube_t * 4u + (s >> 2) < pp.gt && cube_y * 4u + (s & 3u) < pp.gh;
-                    const uint32_t w[4] = {o.x, o.y, o.z, o.w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        acc[2 * e] += ok ? bf16_lo(w[e]) : 0.0f;
-                        acc[2 * e + 1] += ok ? bf16_hi(w[e]) : 0.0f;
-                    }
-                }
-            }
-            // (dx 0 + dx 1) + (dx 2 + dx 3), as cube_pool_kernel's two lane exchanges combine them.
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                if (dx == 0u)
-                    p01[e] = acc[e];
-                else if (dx == 1u)
-                    p01[e] += acc[e];
-                else if (dx == 2u)
-                    p2[e] = acc[e];
-                else
-                    p01[e] += p2[e] + acc[e];
+            for (int e = 0; e < 4; ++e) {
+                acc[2 * e] += ok ? bf16_lo(w[e]) : 0.0f;
+                acc[2 * e + 1] += ok ? bf16_hi(w[e]) : 0.0f;
             }
         }
-        if (live && kind < 2u) {
-            float4* o = reinterpret_cast<float4*>((kind == 0u ? pp.qc : pp.kc) + (uint64_t(h) * pp.cubes + c) * 128u +
-                                                  part * 8u);
-            o[0] = float4{p01[0] / n, p01[1] / n, p01[2] / n, p01[3] / n};
-            o[1] = float4{p01[4] / n, p01[5] / n, p01[6] / n, p01[7] / n};
-        }
+    }
+    // (dx 0 + dx 1) + (dx 2 + dx 3), as cube_pool_kernel's two lane exchanges combine them.
+    if (kind < 2u) {
+        sums[tid] = float4{acc[0], acc[1], acc[2], acc[3]};
+        sums[kPoolThreads + tid] = float4{acc[4], acc[5], acc[6], acc[7]};
+    }
+    __syncthreads();
+    if (live && kind < 2u && dx < 2u) {
+        const float4* a = sums + dx * kPoolThreads + (tid & ~255u) + lane;
+        const float4 a0 = a[0], a1 = a[64], a2 = a[128], a3 = a[192];
+        float4* o = reinterpret_cast<float4*>((kind == 0u ? pp.qc : pp.kc) + (uint64_t(h) * pp.cubes + c) * 128u +
+                                              part * 8u);
+        o[dx] = float4{((a0.x + a1.x) + (a2.x + a3.x)) / n, ((a0.y + a1.y) + (a2.y + a3.y)) / n,
+                       ((a0.z + a1.z) + (a2.z + a3.z)) / n, ((a0.w + a1.w) + (a2.w + a3.w)) / n};
     }
 }
 
@@ -388,23 +411,8 @@ int heads_setup(const MH3HeadsArgs* args, const uint16_t* qkv, const float* q_w,
     p.rows_per_block = std::max(2u, kSlots / p.per_row);
     p.div_row = FastDiv::make(p.per_row);
     p.div_heads = FastDiv::make(a.heads);
+    p.div_half = FastDiv::make(std::max(p.half, 1u));
     return MH3_OK;
-}
-
-// heads_kernel over output rows [row_begin, row_end).
-int launch_heads(HeadsParams p, uint32_t row_begin, uint32_t row_end, hipStream_t stream)
-{
-    if (row_end <= row_begin)
-        return MH3_OK;
-    p.row_begin = row_begin, p.rows = row_end;
-    const uint64_t blocks = (uint64_t(row_end - row_begin) + p.rows_per_block - 1) / p.rows_per_block;
-    size_t lds = (256u + ((p.rows_per_block + 3u) & ~3u) + 2u * size_t(p.rows_per_block) * p.half) * sizeof(float);
-    if (lds < kHeadsLdsFloor)
-        lds = kHeadsLdsFloor;
-    if (const hipError_t e = host::allow_dynamic_lds(reinterpret_cast<const void*>(&heads_kernel), lds); e != hipSuccess)
-        return host::hip_error(e);
-    hipLaunchKernelGGL(heads_kernel, dim3(uint32_t(blocks)), dim3(kHeadsThreads), lds, stream, p);
-    return host::check_launch();
 }
 
 } // namespace
@@ -417,7 +425,15 @@ extern "C" int mh3_heads_partial(const MH3HeadsArgs* args, const uint16_t* qkv, 
     const int rc = heads_setup(args, qkv, q_w, k_w, cos_t, sin_t, map, q, k, v, p);
     if (rc != MH3_OK || args->rows == 0)
         return rc;
-    return launch_heads(p, 0u, args->rows, static_cast<hipStream_t>(stream));
+    const uint64_t blocks = (uint64_t(p.rows) + p.rows_per_block - 1) / p.rows_per_block;
+    size_t lds = (256u + ((p.rows_per_block + 3u) & ~3u) + 2u * size_t(p.rows_per_block) * p.half) * sizeof(float);
+    if (lds < kHeadsLdsFloor)
+        lds = kHeadsLdsFloor;
+    if (const hipError_t e = host::allow_dynamic_lds(reinterpret_cast<const void*>(&heads_kernel), lds); e != hipSuccess)
+        return host::hip_error(e);
+    hipLaunchKernelGGL(heads_kernel, dim3(uint32_t(blocks)), dim3(kHeadsThreads), lds, static_cast<hipStream_t>(stream),
+                       p);
+    return host::check_launch();
 }
 
 extern "C" int mh3_heads_partial_pool(const MH3HeadsArgs* args, const MH3CubeArgs* cubes, const uint16_t* qkv,
@@ -462,21 +478,19 @@ extern "C" int mh3_heads_partial_pool(const MH3HeadsArgs* args, const MH3CubeArg
         if (host::any_overlap(in, out))
             return MH3_ERR_PARAM;
     }
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    const uint32_t video0 = uint32_t(cb.row0), video1 = uint32_t(cb.row0 + span);
-    int r = launch_heads(p, 0u, video0, st); // rows before the cubes, and after them (the dense rows)
-    if (r == MH3_OK)
-        r = launch_heads(p, video1, args->rows, st);
-    if (r != MH3_OK)
-        return r;
     HeadsPoolParams pp{};
     pp.hp = p, pp.qc = qc, pp.kc = kc, pp.counts = counts, pp.row0 = cb.row0;
     pp.gt = cb.grid_t, pp.gh = cb.grid_h, pp.gw = cb.grid_w, pp.cw = (cb.grid_w + 3u) / 4u;
     pp.plane = ((cb.grid_h + 3u) / 4u) * pp.cw, pp.cubes = uint32_t(ncubes), pp.grid = grid ? 1u : 0u;
-    const size_t lds = (256u + 64u + 2u * std::max(64u * p.half, 8u)) * sizeof(float); // 26 KB at rot 96
+    pp.parts = (p.per_row + 7u) / 8u;
+    pp.video0 = uint32_t(cb.row0), pp.video1 = uint32_t(cb.row0 + span);
+    pp.cube_wgs = uint32_t(ncubes) * pp.parts;
+    pp.wgs0 = (pp.video0 + p.rows_per_block - 1u) / p.rows_per_block;
+    const uint64_t wgs = uint64_t(pp.cube_wgs) + pp.wgs0 + (p.rows - pp.video1 + p.rows_per_block - 1u) / p.rows_per_block;
+    const size_t lds = (256u + 64u + 2u * std::max(64u * p.half, 8u) + 8u * kPoolThreads) * sizeof(float); // 26 KB at rot 96
     if (const hipError_t e = host::allow_dynamic_lds(reinterpret_cast<const void*>(&heads_pool_kernel), lds);
         e != hipSuccess)
         return host::hip_error(e);
-    hipLaunchKernelGGL(heads_pool_kernel, dim3(uint32_t(ncubes)), dim3(kPoolThreads), lds, st, pp);
+    hipLaunchKernelGGL(heads_pool_kernel, dim3(uint32_t(wgs)), dim3(kPoolThreads), lds, static_cast<hipStream_t>(stream), pp);
     return host::check_launch();
 }

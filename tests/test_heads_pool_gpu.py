@@ -149,3 +149,22 @@ def test_heads_partial_pool_grid_layout_768p(dev):
     torch.cuda.synchronize()
     for name, a, b in zip(("q", "k", "v", "qc", "kc"), got, (q, k, v, qc, kc)):
         assert same(a, b), f"{name} differs at 768p (grid layout)"
+
+
+@pytest.mark.parametrize("grid,heads,n_before,n_after,with_v", [((1, 17, 30), 56, 0, 35, True), ((2, 5, 7), 7, 3, 1, True),
+                                                                ((5, 12, 20), 40, 0, 77, True), ((6, 4, 9), 3, 50, 0, False)])
+def test_heads_partial_pool_grid_layout_edges(dev, grid, heads, n_before, n_after, with_v):
+    """The model's row order with frames of slots past the grid's edge, head vectors that do not fill the last
+    workgroup's 8 (21, 9, 6 of them a row), and rows before and after the grid's in the same launch: bit for bit the
+    two kernels, into outputs filled with NaN."""
+    video = grid[0] * grid[1] * grid[2]
+    rows = n_before + video + n_after
+    x, qw, kw, ct, st = inputs(dev, rows, heads, 96, seed=heads)
+    q, k, v = mh.heads_partial(x, heads, qw, kw, ct, st, with_v=with_v, layout="rows")
+    a = mh.cube_args(heads, grid, row0=n_before, head_stride=128, row_stride=heads * 128)
+    want = (q, k, v, *mh.cube_pool(a, q, k))
+    bufs = [torch.full((rows, heads * 128), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(3)]
+    got = mh.heads_partial_pool(x, heads, grid, qw, kw, ct, st, with_v=with_v, layout="rows", row0=n_before,
+                                cube_layout=mh.CUBES_GRID, q=bufs[0], k=bufs[1], v=bufs[2] if with_v else None)
+    for name, g, w in zip(("q", "k", "v", "qc", "kc"), got, want):
+        assert same(g, w), name

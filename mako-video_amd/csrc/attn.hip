@@ -49,7 +49,7 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t kAttnThreads = 128;
-constexpr bool kAttnXcd = true;   // map each XCD to a contiguous eighth of every head's query cubes
+
 constexpr bool kAttnSweep = true; // rotate each cube tile's pass list so an XCD's resident tiles sweep the keys together
 constexpr uint32_t kAttnInStep = 4; // rounds of an XCD's cube tiles that walk their lists unrotated (1, 2, 8: slower;
                                     // 3, 5, 6: within 1%)
@@ -68,8 +68,10 @@ struct AttnParams {
     uint32_t gt, gh, gw, ch, cw, plane; // plane = ch * cw cubes a frame group
     uint32_t cubes, heads, n_dense, nd; // nd: dense tiles of 64 rows
     uint32_t layout, out_stride;
-    uint32_t xcd_slices; // cube tiles mapped to XCDs in eighths of each head (needs 8 | cubes and 8 | nd heads)
-    uint32_t sweep;      // with xcd_slices: cube workgroups an XCD runs at once (0: pass lists in plain order)
+    // The workgroup-to-tile map: `share` XCDs take a head's cube tiles in contiguous parts of `per`, `groups` = 8 / share
+    // heads run at once; XCD x takes the dense tiles x dense_per .. of all heads' in turn.
+    uint32_t share, groups, per, dense_per;
+    uint32_t sweep; // cube workgroups an XCD runs at once (0: pass lists in plain order)
     FastDiv div_plane, div_cw; // c / plane and c / cw by multiply-high: a key tile's cube coordinates cost a few
                                // scalar instructions instead of integer divisions
     float scale_log2;    // score scale times log2(e): softmax in base 2
@@ -175,31 +177,27 @@ __global__ __launch_bounds__(kAttnThreads, STAGES == 2 ? 1 : 2) void attn_sparse
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
 
     // This workgroup's head and query tile: the dense query tiles of every head first, then the cube tiles. Blocks
-    // go to the 8 XCDs round-robin (block b to XCD b % 8); when the counts allow, XCD x takes the x-th eighth of each
-    // head's cubes in raster order (or in p.order's), so the workgroups resident on one XCD are query cubes whose
-    // pass lists overlap and meet in that XCD's L2, while all XCDs stay on the same head.
+    // go to the 8 XCDs round-robin (block b to XCD b % 8). An XCD takes a contiguous part of a head's cubes in raster
+    // order (or in p.order's), so the workgroups resident on it are query cubes whose pass lists overlap and meet in
+    // its L2; how many XCDs share a head is the host's choice (share_of).
     uint32_t h, qt, rank = 0; // rank: the workgroup's place in its XCD's sequence of cube tiles
     {
-        const uint32_t b = blockIdx.x, dense_blocks = p.nd * p.heads;
+        const uint32_t b = blockIdx.x, x = b % 8u, dense_blocks = 8u * p.dense_per;
         if (b < dense_blocks) {
-            // With the XCD slices, XCD x takes the dense tiles of whole heads (the x-th eighth of them in order), so
-            // a head's dense tiles, which walk the same keys in the same order, share each K/V tile in one L2 (5
+            const uint32_t l = x * p.dense_per + b / 8u;
+            // A head's dense tiles, which walk the same keys in the same order, share each K/V tile in one L2 (5
             // heads at 768p: 7.29-7.32 ms against 7.47-7.48 with a head's tiles dealt over the 8 XCDs).
-            const uint32_t l = p.xcd_slices ? (b % 8u) * (dense_blocks / 8u) + b / 8u : b;
+            if (l >= p.nd * p.heads)
+                return;
             h = l / p.nd;
             qt = l - h * p.nd;
         } else {
-            const uint32_t r = b - dense_blocks;
-            uint32_t j; // the cube tile's place among its head's
-            if (p.xcd_slices) {
-                const uint32_t per = p.cubes / 8u, k = r / 8u;
-                h = k / per;
-                j = (r % 8u) * per + (k - h * per);
-                rank = k;
-            } else {
-                h = r / p.cubes;
-                j = r - h * p.cubes;
-            }
+            const uint32_t k = (b - dense_blocks) / 8u, round = k / p.per;
+            h = round * p.groups + x / p.share;
+            const uint32_t j = (x % p.share) * p.per + (k - round * p.per); // the cube tile's place among its head's
+            if (h >= p.heads || j >= p.cubes)
+                return;
+            rank = k;
             qt = p.nd + (p.order ? min(uint32_t(p.order[uint64_t(h) * p.cubes + j]), p.cubes - 1u) : j);
         }
     }
@@ -422,6 +420,20 @@ __global__ __launch_bounds__(kAttnThreads, STAGES == 2 ? 1 : 2) void attn_sparse
 
 namespace {
 
+// How many XCDs share one head's cube tiles (8, 4, 2 or 1), `bytes` being a head's K and V. Fewer XCDs a head mean more
+// of its query cubes on each L2 at once, over the same keys (56 heads, 33 x 15 x 35, 9 MB a head: 3.90 ms at 8, 3.72 at
+// 2 and 1; the dense 37 x 17 x 30: 23.2 and 22.5), but 8 / share heads' K and V in flight at once: past half of the
+// 256 MB MALL that begins to cost (40 heads of 66 MB, independent and overlapping lists: 53.0 and 49.4 ms at 8, 50.2
+// and 48.8 at 4, 49.0 and 50.2 at 2, 49.1 and 51.9 at 1). The heads must also divide over the groups (5 heads of 66 MB:
+// 6.7 ms at 8, 7.9 at 4, 9.4 at 1).
+uint32_t share_of(uint32_t heads, uint64_t bytes)
+{
+    uint32_t share = 1;
+    while (share < 8u && (heads % (8u / share) != 0 || 8u / share * bytes > (144ull << 20)))
+        share *= 2u;
+    return share;
+}
+
 // order: null for the plain entry point; `ordered`: the ordered one, which needs it.
 int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, const uint16_t* v, const int32_t* idx,
                 const int32_t* cnt, const int32_t* order, bool ordered, uint16_t* out, mh3_stream_t stream)
@@ -483,16 +495,17 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     p.div_plane = FastDiv::make(p.plane);
     p.div_cw = FastDiv::make(p.cw);
     p.nd = uint32_t(nd), p.layout = c.layout, p.out_stride = c.out_stride;
-    p.xcd_slices = kAttnXcd && cubes % 8u == 0 && (nd * c.heads) % 8u == 0 ? 1u : 0u;
+    p.share = share_of(c.heads, (video + args->n_dense) * 512ull);
+    p.groups = 8u / p.share, p.per = (p.cubes + p.share - 1u) / p.share, p.dense_per = (p.nd * p.heads + 7u) / 8u;
     const float scale = args->scale > 0.0f ? args->scale : 0.08838834764831845f; // 1 / sqrt(128)
     p.scale_log2 = scale * 1.4426950408889634f;
-    const uint64_t blocks = (cubes + nd) * c.heads;
+    const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
     constexpr int kStages = kAttnStages;
     const void* kern = reinterpret_cast<const void*>(&attn_sparse_kernel<kStages>);
     const size_t lds = size_t(kStages) * kStageBytes;
     if (const hipError_t e = host::allow_dynamic_lds(kern, lds); e != hipSuccess)
         return host::hip_error(e);
-    if (kAttnSweep && p.xcd_slices) {
+    if (kAttnSweep) {
         int per_cu = 0;
         if (const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, int(kAttnThreads), lds);
             e != hipSuccess)

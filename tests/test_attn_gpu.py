@@ -317,3 +317,30 @@ def test_flash_attn_sparse_768p_40_heads(dev, ordered):
     for (h, tile), (lh, _) in zip(tiles, local):
         r = orc.attn_tile_rows(grid, orc.CUBES_GRID, 0, video, n_dense, tile)
         check(ob[lh, r], want[lh, r], f"768p 40 heads: head {h} tile {tile}")
+
+
+@pytest.mark.parametrize("heads,grid,layout,n_dense", [
+    (8, (7, 9, 10), orc.CUBES_GRID, 70),        # an XCD a head; 18 cubes
+    (12, (5, 9, 13), orc.CUBES_GATHERED, 130),  # two XCDs a head, 24 cubes in halves of 12
+    (6, (5, 12, 9), orc.CUBES_GRID, 0),         # four XCDs a head, 18 cubes in parts of 5; no dense tiles
+    (5, (3, 5, 9), orc.CUBES_GRID, 200),        # eight XCDs a head, 6 cubes: parts of one, two of them empty
+    (16, (1, 4, 4), orc.CUBES_GATHERED, 3),     # one cube a head
+])
+def test_flash_attn_sparse_heads_over_the_xcds(dev, heads, grid, layout, n_dense):
+    """Every way the heads and their cubes fall on the XCDs, with parts that do not divide: every row of every head
+    against the float32 restatement, into a NaN-filled output."""
+    C = orc.cube_count(*grid)
+    video = C * 64 if layout == orc.CUBES_GATHERED else grid[0] * grid[1] * grid[2]
+    rows = video + n_dense
+    g = torch.Generator(device=dev).manual_seed(heads)
+    q, k, v = [torch.randn((heads, rows, 128), generator=g, device=dev).to(torch.bfloat16) for _ in range(3)]
+    rng = np.random.default_rng(heads)
+    kk = max(1, C // 3)
+    idx, cnt = (torch.from_numpy(x).to(dev) for x in
+                orc.cube_topk(rng.standard_normal((heads, C, C)), grid, kk, 1, out_stride=kk + 2))
+    a = mh.cube_args(heads, grid, layout=layout, head_stride=rows * 128, out_stride=kk + 2)
+    for order in (None, mh.cube_order(a, idx, cnt)):
+        out = mh.flash_attn_sparse_128(a, q, k, v, idx, cnt, dense_row0=video, n_dense=n_dense,
+                                       out=nan_filled((heads, rows, 128), dev), order=order)
+        ref = attn_sparse_f32(q, k, v, idx, cnt, grid, video, n_dense, layout=layout)
+        check_attn_f32(out, ref, f"{heads} heads {grid}")

@@ -2,17 +2,18 @@
 // out = silu(x Wg sg) * (x Wu su), replacing the reference's `gemm_i8` + `swiglu_rows` pair for fc1 (mako-common;
 // docs/performance.md:120-136, docs/architecture.md:65: fc1's [gate; value] rows, then SwiGLU). The same kernel with
 // bf16 weights is the dense fc1 of the `--int8 none` path (the reference's bf16 `Gemm::encode`,
-// docs/performance.md:52-69): its B tiles then stream into LDS like A's, one K-step ahead, and there is no scale.
+// docs/performance.md:52-69): its B tiles then stream into LDS like A's, and there is no scale.
 // With int8 x as well (W8A8, the reference's own `gemm_i8`: activations quantized per row) both operands stream
 // into LDS and the int8 MFMA (v_mfma_i32_16x16x64_i8, exact int32 sums) takes 128 k a K-step; the epilogue applies
 // both scales. Two more epilogues make the same kernel the qkv projection (a plain store) and the out and fc2
 // projections (gate_add_rows folded in: the residual += gate * y, in place).
 //
 // Design (gfx950, v_mfma_f32_16x16x32_bf16):
-// - A workgroup of 8 wavefronts (2 along rows x 4 along columns) computes a 256-row x 128-column output tile, i.e.
-//   the 128 gate columns [n0, n0+128) and the 128 up columns [n + n0, n + n0 + 128) of y, so the SwiGLU epilogue has
-//   both halves in registers. Each wave owns 128 rows x (32 gate + 32 up) columns: 8 x 4 MFMA tiles of 16 x 16.
-// - K advances 64 at a time. A (x, bf16) streams from HBM straight into a 3-stage LDS ring with buffer loads that
+// - A workgroup of 8 wavefronts (2 along rows x 4 along columns) computes a tile of BM = 256 rows (fewer where a call
+//   has too few rows to fill the chip with those: row_tile) x 128 columns, i.e. the 128 gate columns [n0, n0+128) and
+//   the 128 up columns [n + n0, n + n0 + 128) of y, so the SwiGLU epilogue has both halves in registers. Each wave
+//   owns BM / 2 rows x (32 gate + 32 up) columns, at 256 rows 8 x 4 MFMA tiles of 16 x 16.
+// - K advances 64 at a time. A (x, bf16) streams from HBM straight into an LDS ring (3 stages) with buffer loads that
 //   write LDS (no VGPR round trip); B (int8 w) is loaded as 16-byte vectors into registers one K-step ahead and
 //   widened to bf16 into a 2-stage LDS ring (exact: |w| <= 127 fits bf16's 8-bit significand), so dequantization
 //   costs no extra HBM traffic and the scale is applied once to the float accumulator in the epilogue:
@@ -31,6 +32,7 @@
 //   nothing hides the fragment reads and the barrier.
 #include "mh3_common.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace mh3 {
@@ -38,12 +40,19 @@ namespace mh3 {
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-constexpr uint32_t kBM = 256, kBN = 128, kBK = 64;
-// LDS: a ring of 3 A stages (256 rows x 64 k bf16 = 2048 16-byte chunks each), then 2 B stages (256 B-rows x 64 k,
-// widened to bf16: 2048 chunks each): 160 KiB, gfx950's whole LDS.
-constexpr uint32_t kStageChunks = 2048, kAStages = 3, kBStages = 2;
-constexpr uint32_t kBBase = kAStages * kStageChunks;
-constexpr size_t kGemmLds = size_t(kAStages + kBStages) * kStageChunks * 16;
+constexpr uint32_t kBM = 256, kBN = 128, kBK = 64; // kBM: the largest row tile
+// LDS: a ring of A stages (BM rows x 64 k bf16: 8 16-byte chunks a row), then B stages (256 B-rows x 64 k, bf16 or
+// widened to it: 2048 chunks each). 3 A and 2 B stages fill gfx950's 160 KiB at 256 rows. A smaller row tile spends less
+// time on a K-step than a load takes to arrive, so where both operands stream into LDS it takes more stages and its
+// loads go out further ahead (128 rows, x [1277][14336] bf16, 21 column tiles: 249 us with 3 and 2, 208 with 4 and 3).
+constexpr uint32_t kBChunks = 2048;
+template <int BM, bool I8>
+struct GemmRing {
+    static constexpr uint32_t kAChunks = BM * 8u;
+    static constexpr uint32_t kAStages = BM <= 128 && !I8 ? 4 : 3;
+    static constexpr uint32_t kBStages = I8 ? 2 : BM <= 64 ? 4 : BM <= 128 ? 3 : 2;
+    static constexpr size_t kBytes = (size_t(kAStages) * kAChunks + size_t(kBStages) * kBChunks) * 16;
+};
 constexpr uint32_t kBandM = 4; // row tiles an XCD sweeps across all column tiles before moving on
 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
@@ -76,13 +85,15 @@ __device__ __forceinline__ u32x4_t widen8(uint32_t w0, uint32_t w1)
     return r;
 }
 
+template <int BM>
 __device__ __forceinline__ void tile_of(uint32_t mt, uint32_t nt, uint32_t& tm, uint32_t& tn)
 {
+    constexpr uint32_t kBand = kBandM * kBM / uint32_t(BM);
     const uint32_t nb = gridDim.x, b = blockIdx.x;
     const uint32_t logical = (nb % 8u == 0u) ? (b % 8u) * (nb / 8u) + b / 8u : b;
-    const uint32_t band = logical / (kBandM * nt), within = logical - band * kBandM * nt;
-    const uint32_t in_band = min(kBandM, mt - band * kBandM);
-    tm = band * kBandM + within % in_band;
+    const uint32_t band = logical / (kBand * nt), within = logical - band * kBand * nt;
+    const uint32_t in_band = min(kBand, mt - band * kBand);
+    tm = band * kBand + within % in_band;
     tn = within / in_band;
 }
 
@@ -132,7 +143,7 @@ typedef int int32x4 __attribute__((ext_vector_type(4)));
 // tile (the two half-waves' rows, 4 apart, fall on disjoint banks); then each thread takes 8 consecutive columns of
 // a row, so the output, and with kGateAdd the residual, moves in 16-byte accesses, 16 threads to a row's 256 bytes.
 // The results round to bf16 once, at the end, as they would written straight from the registers.
-template <int WM, int WN, int MODE, int EPI, int TM, int TN, typename Acc>
+template <int BM, int WM, int WN, int MODE, int EPI, int TM, int TN, typename Acc>
 __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* smem, uint32_t M, uint32_t N,
                                               uint32_t m0, uint32_t w_lo, uint32_t w_hi,
                                               const float* __restrict__ scale, const float* __restrict__ xscale,
@@ -142,7 +153,7 @@ __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* s
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, wm = wave / WN, wn = wave % WN;
     const uint32_t rl = lane % 16u;
     constexpr uint32_t kEpiStride = kBN + 8u; // floats a staged row: 4 rows apart = 32 banks apart
-    static_assert(kBM * kEpiStride * sizeof(float) <= kGemmLds, "the staged half-tile fits in the LDS");
+    static_assert(BM * kEpiStride * sizeof(float) <= GemmRing<BM, MODE == 0>::kBytes, "the staged half-tile fits in the LDS");
     constexpr int kHalves = EPI == kSwiGLU ? 1 : 2;
     float* const stage = reinterpret_cast<float*>(smem);
     lds_barrier(); // every wave is done with the last K-step's fragments
@@ -158,7 +169,7 @@ __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* s
             for (int a = 0; a < TM; ++a) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const uint32_t r = wm * (kBM / WM) + uint32_t(a) * 16u + 4u * (lane >> 4) + uint32_t(e);
+                    const uint32_t r = wm * (uint32_t(BM) / WM) + uint32_t(a) * 16u + 4u * (lane >> 4) + uint32_t(e);
                     const float sx = MODE == kW8A8 ? xscale[min(m0 + r, M - 1u)] : 1.0f;
                     float v;
                     if constexpr (EPI == kSwiGLU) {
@@ -174,7 +185,7 @@ __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* s
         lds_barrier();
         // Output column of staged column 0: the tile's gate columns (SwiGLU), else its first or second 128 columns.
         const uint32_t col0 = hv == 0 ? w_lo : w_hi;
-        for (uint32_t q = tid; q < kBM * 16u; q += kThreads) {
+        for (uint32_t q = tid; q < uint32_t(BM) * 16u; q += kThreads) {
             const uint32_t r = q >> 4, c8 = (q & 15u) * 8u, row = m0 + r;
             if (row >= M)
                 break; // rows grow with q
@@ -214,7 +225,7 @@ __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* s
 // (16 columns each, from wn * 16 TN) and the TN matching up column tiles, on 16 x 16 MFMA tiles
 // (v_mfma_f32_16x16x32_bf16, v_mfma_i32_16x16x64_i8). Every LDS row holds 128 bytes of k: 64 k of bf16 or 128 k of
 // int8, so a K-step is 64 or 128 k.
-template <int WM, int WN, int MODE, int EPI>
+template <int BM, int WM, int WN, int MODE, int EPI>
 __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     const void* __restrict__ xv, const void* __restrict__ wv, const float* __restrict__ scale,
     const float* __restrict__ xscale, uint16_t* __restrict__ out, uint32_t M, uint32_t N, uint32_t K, uint32_t mt,
@@ -226,14 +237,17 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     constexpr uint32_t kKS = 128u / kEA;                  // k of a K-step
     using Acc = typename std::conditional<MODE == kW8A8, int32x4, floatx4>::type;
     constexpr uint32_t kThreads = WM * WN * 64, kWaves = WM * WN;
-    constexpr int TM = int(kBM / WM / 16), TN = int(kBN / WN / 16); // MFMA tiles: rows, and gate (= up) columns
+    constexpr int TM = int(BM / WM / 16), TN = int(kBN / WN / 16); // MFMA tiles: rows, and gate (= up) columns
     // Row tiles whose A fragments a sub-step holds: half of them (a sub-step is one 32-k half of the K-step over one
     // half of the wave's rows).
     constexpr int FA = TM / 2;
     extern __shared__ u32x4_t smem[];
+    using Ring = GemmRing<BM, I8>;
+    constexpr uint32_t kAChunks = Ring::kAChunks, kAStages = Ring::kAStages, kBStages = Ring::kBStages;
+    constexpr uint32_t kBBase = kAStages * kAChunks;
     uint32_t tm, tn;
-    tile_of(mt, nt, tm, tn);
-    const uint32_t m0 = tm * kBM;
+    tile_of<BM>(mt, nt, tm, tn);
+    const uint32_t m0 = tm * uint32_t(BM);
     // The tile's two 128-row halves of w (and the output columns they give): gate and up rows, or consecutive rows.
     const uint32_t w_lo = EPI == kSwiGLU ? tn * kBN : tn * 2u * kBN;
     const uint32_t w_hi = EPI == kSwiGLU ? N + w_lo : w_lo + kBN;
@@ -245,7 +259,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     // wave fills 2048 / kWaves of them, 64 a instruction; lane L of instruction i lands in chunk q = (wave * AI + i) *
     // 64 + L = row * 8 + physical chunk and fetches the logical chunk the swizzle puts there. The descriptor starts
     // at this tile's first row; rows past M read zero.
-    constexpr int AI = int(kStageChunks / 64 / kWaves);
+    constexpr int AI = int(kAChunks / 64 / kWaves), BD = int(kBChunks / 64 / kWaves);
     const uint64_t a_left = uint64_t(M - m0) * K * kEA;
     const __amdgpu_buffer_rsrc_t ra = buffer_rsrc(reinterpret_cast<const char*>(xv) + uint64_t(m0) * K * kEA,
                                                   uint32_t(a_left < 0x7fffffffu ? a_left : 0x7fffffffu));
@@ -257,7 +271,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         a_off[i] = row * K * kEA + c * 16u;
     }
     auto a_issue = [&](uint32_t kt) {
-        u32x4_t* stage = smem + (kt % kAStages) * kStageChunks + wave * AI * 64u;
+        u32x4_t* stage = smem + (kt % kAStages) * kAChunks + wave * AI * 64u;
 #pragma unroll
         for (int i = 0; i < AI; ++i)
             lds_dma16(ra, stage + i * 64, a_off[i], int(kt * 128u));
@@ -290,7 +304,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     u32x4_t rb[BI];
     // Piece p of tile kt's B write: half p % 2 of register chunk p / 2, widened and stored.
     auto b_piece = [&](uint32_t kt, const u32x4_t (&rb)[BI], int p) {
-        char* B = lds + (kBBase + (kt % kBStages) * kStageChunks) * 16u;
+        char* B = lds + (kBBase + (kt % kBStages) * kBChunks) * 16u;
         const int i = p >> 1, h = p & 1;
         *reinterpret_cast<u32x4_t*>(B + (h ? b_hi[i] : b_lo[i])) = widen8(rb[i][2 * h], rb[i][2 * h + 1]);
     };
@@ -301,18 +315,18 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     };
     // bf16 weights, and int8 weights with int8 x: B goes straight into its LDS ring like A, B-row r of the tile from
     // weight row n0 + r (gate) or n + n0 + r - 128 (up), with A's chunk-to-lane assignment and swizzle.
-    uint32_t bd_off[AI];
+    uint32_t bd_off[BD];
 #pragma unroll
-    for (int i = 0; i < AI && !I8; ++i) {
-        const uint32_t row = (wave * AI + uint32_t(i)) * 8u + (lane >> 3);
+    for (int i = 0; i < BD && !I8; ++i) {
+        const uint32_t row = (wave * BD + uint32_t(i)) * 8u + (lane >> 3);
         const uint32_t c = (lane & 7u) ^ ((row >> 1) & 7u);
         const uint32_t wrow = row < kBN ? w_lo + row : w_hi + (row - kBN);
         bd_off[i] = wrow * K * kEB + c * 16u;
     }
     auto b_dma = [&](uint32_t kt) {
-        u32x4_t* stage = smem + kBBase + (kt % kBStages) * kStageChunks + wave * AI * 64u;
+        u32x4_t* stage = smem + kBBase + (kt % kBStages) * kBChunks + wave * BD * 64u;
 #pragma unroll
-        for (int i = 0; i < AI; ++i)
+        for (int i = 0; i < BD; ++i)
             lds_dma16(rw, stage + i * 64, bd_off[i], int(kt * 128u));
     };
 
@@ -322,7 +336,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     // sub-step serves all tiles; t moves it by 16 rows. (The 16 rows a quarter-wave reads at one chunk then cover the
     // 64 banks once.)
     const uint32_t rs = lane % 16u, fsx = (rs >> 1) & 7u;
-    const uint32_t fa_base = (wm * (kBM / WM) + rs) * 128u, fb_base = (wn * 16u * TN + rs) * 128u;
+    const uint32_t fa_base = (wm * uint32_t(BM / WM) + rs) * 128u, fb_base = (wn * 16u * TN + rs) * 128u;
     constexpr uint32_t kRowBytes = 16u * 128u; // one MFMA tile's rows in a stage
     uint32_t fko[4];
 #pragma unroll
@@ -330,13 +344,13 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         fko[ks] = (((ks >> 1) * 4u + (lane >> 4)) ^ fsx) * 16u;
     auto frags_a = [&](uint32_t kt, uint32_t ks, bf16x8_t (&fa)[FA]) {
         const uint32_t t0 = (ks & 1u) * uint32_t(FA);
-        const char* A = lds + (kt % kAStages) * kStageChunks * 16u + fa_base + fko[ks] + t0 * kRowBytes;
+        const char* A = lds + (kt % kAStages) * kAChunks * 16u + fa_base + fko[ks] + t0 * kRowBytes;
 #pragma unroll
         for (int t = 0; t < FA; ++t)
             fa[t] = *reinterpret_cast<const bf16x8_t*>(A + t * kRowBytes);
     };
     auto frags_b = [&](uint32_t kt, uint32_t ks, bf16x8_t (&fb)[2 * TN]) {
-        const char* B = lds + (kBBase + (kt % kBStages) * kStageChunks) * 16u + fb_base + fko[ks];
+        const char* B = lds + (kBBase + (kt % kBStages) * kBChunks) * 16u + fb_base + fko[ks];
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
             fb[t] = *reinterpret_cast<const bf16x8_t*>(B + t * kRowBytes);
@@ -392,7 +406,16 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         }
     };
 
-    // Prologue: tile 0's B widened into LDS and tile 0's A in LDS; tile 1's B in registers and A in flight to LDS.
+    // How many K-steps A's loads, and those of a B that streams into LDS, go out ahead.
+    constexpr uint32_t DA = kAStages - 1u, DB = kBStages - 1u;
+    // Whether such a B goes out right after the barrier, or after the last sub-step's MFMAs have issued: a quarter of a
+    // K-step earlier, but between the fragment reads and the MFMAs. At 256 rows the MFMAs set the pace (19,305 x 5376 ->
+    // 28,672: 4.72 ms early, 4.63 late); with fewer the loads do.
+    constexpr bool kEarlyB = !I8 && BM <= 128;
+    static_assert(DA == DB || DA == DB + 1u, "the order that the waits below count on");
+    static_assert(kEarlyB || (DA == 2 && DB == 1));
+    // Prologue: tile 0 in LDS (its B widened), and the later tiles' loads in flight: with int8 weights tile 1's B to
+    // registers and A to LDS; with kEarlyB tiles 1 .. DB's B and 1 .. DA - 1's A, otherwise tile 1's A.
     // The explicit wait is needed: the compiler may issue the B loads ahead of the LDS-bound A loads, and then the
     // waits it places for the B registers leave tile 0's A outstanding.
     a_issue(0);
@@ -401,11 +424,24 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     else
         b_dma(0);
     __builtin_amdgcn_sched_barrier(0);
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    if constexpr (kEarlyB) {
+#pragma unroll
+        for (uint32_t t = 1; t <= DB; ++t) {
+            if (t < KT)
+                b_dma(t);
+            if (t < DA && t < KT)
+                a_issue(t);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    if (kEarlyB && KT > DA) // the loads after tile 0's
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(int(DB) * BD + int(DA - 1u) * AI));
+    else
+        __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (I8)
         b_write(0, rb);
-    if (KT > 1) {
+    if (!kEarlyB && KT > 1) {
         if constexpr (I8)
             b_issue(1, rb);
         a_issue(1);
@@ -418,20 +454,21 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     bf16x8_t fa[2][FA], fb[2][2 * TN];
     frags(0, 0, fa[0], fb[0]);
 
-    // One K-step over tile kt (four sub-steps of 16 k). Tile kt+1's B is widened from registers into LDS in four
-    // pieces placed between the MFMAs of the first two sub-steps. Then the wave waits for everything it has in
-    // flight (tile kt+1's A, issued a step ago) and tile kt+2's B and A loads go out. The barrier publishing tile kt+1
-    // comes after the third sub-step's MFMAs, and
-    // the fourth sub-step's operands are already in registers: the MFMAs keep running while tile kt+1's first
-    // fragments load. LDS stages written in step kt (A stage (kt+2) % 3, B stage (kt+1) % 2) were last read before
-    // step kt-1's barrier. The last step is a separate instance (kLast) so that the loop body has no branch around
-    // the barrier: at such a join the compiler's LDS wait would also cover tile kt+1's fragment reads.
+    // One K-step over tile kt (four sub-steps). With int8 weights, tile kt+1's B is widened from registers into LDS in
+    // pieces placed between the MFMAs of the first two sub-steps; then the wave waits for everything it has in flight
+    // (tile kt+1's A, issued a step ago) and tile kt+2's B goes out. Tile kt+DA's A goes out there too. The barrier
+    // publishing tile kt+1 comes after the third sub-step's MFMAs, and the fourth sub-step's operands are already in
+    // registers: the MFMAs keep running while tile kt+1's first fragments load. A B that streams into LDS goes out
+    // after the barrier (kEarlyB) or the step's last MFMAs, DB steps ahead. LDS stages written after step kt-1's barrier (A's (kt+DA) % kAStages, B's
+    // (kt+DB) % kBStages) were last read before it. The last step is a separate instance (kLast) so that the loop body
+    // has no branch around the barrier: at such a join the compiler's LDS wait would also cover tile kt+1's fragment
+    // reads.
     // B sets of sub-steps 0..3: one a k-half (0, 0, 1, 1).
     constexpr int B1 = 0, B2 = 1, B3 = 1;
     auto kstep = [&](uint32_t kt, auto last) {
         constexpr bool kLast = decltype(last)::value;
-        if constexpr (!I8 && !kLast)
-            b_dma(kt + 1); // into B stage (kt+1) % 2, last read before step kt-1's barrier
+        if constexpr (!I8 && !kEarlyB && !kLast)
+            b_dma(kt + 1); // DB is 1
         frags(kt, 1, fa[1], fb[B1]);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (kLast || !I8)
@@ -447,13 +484,12 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         if constexpr (!kLast) {
             if constexpr (I8) {
                 __builtin_amdgcn_s_waitcnt(waitcnt_vm(0)); // tile kt+1's A complete too
-                if (kt + 2 < KT) {
+                if (kt + 2 < KT)
                     b_issue(kt + 2, rb);
-                    a_issue(kt + 2);
-                }
-            } else if (kt + 2 < KT) {
-                a_issue(kt + 2);
             }
+            if (kt + DA < KT)
+                a_issue(kt + DA);
+            __builtin_amdgcn_sched_barrier(0); // the waits count these loads: none moves past here
         }
         frags(kt, 3, fa[1], fb[B3]);
         __builtin_amdgcn_sched_barrier(0);
@@ -461,14 +497,18 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (!kLast) {
             if constexpr (!I8) {
-                // Loads complete in order: all but tile kt+2's AI A loads means tile kt+1's A and B are in LDS.
-                if (kt + 2 < KT)
-                    __builtin_amdgcn_s_waitcnt(waitcnt_vm(AI));
+                // Loads complete in order: tile kt+1 is in LDS once only the later tiles' loads are left, the B of
+                // DB - 1 tiles and the A of DB - 1 (DB, where A goes out a step before B).
+                if (kt + DA < KT)
+                    __builtin_amdgcn_s_waitcnt(waitcnt_vm(int(DB - 1u) * (BD + AI) + (DA > DB ? AI : 0)));
                 else
                     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
             }
             lds_barrier();
             frags(kt + 1, 0, fa[0], fb[0]);
+            if constexpr (kEarlyB)
+                if (kt + 1u + DB < KT)
+                    b_dma(kt + 1u + DB); // into the stage that tile kt's B leaves: every wave has read it
         }
         __builtin_amdgcn_sched_barrier(0);
         mfmas(3, fa[1], fb[B3]);
@@ -477,12 +517,51 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         kstep(kt, std::false_type{});
     kstep(KT - 1, std::true_type{});
 
-    gemm_epilogue<WM, WN, MODE, EPI, TM, TN>(acc, smem, M, N, m0, w_lo, w_hi, scale, xscale, out, gg);
+    gemm_epilogue<BM, WM, WN, MODE, EPI, TM, TN>(acc, smem, M, N, m0, w_lo, w_hi, scale, xscale, out, gg);
 }
 
 } // namespace mh3
 
 namespace {
+
+// The row tile of a launch of m rows and nt column tiles: the one whose rounds over the CUs (one workgroup each) take
+// least, the larger of equals. `time` is a round's cost against 256 rows': it falls more slowly than the rows, since a
+// K-step streams the same B and has the same chain of loads, barrier and fragment reads. Measured a K-step at K 14336,
+// bf16, rounds of the whole chip: 1.55, 1.36, 1.05 and 0.68 us at 256, 192, 128 and 64 rows, and on a nearly empty chip
+// 1.27, 1.08, 0.87 and 0.76. Chosen against 256 rows (us): 945 x 14336 -> 5376 bf16 284 -> 186, int8 weights 313 ->
+// 214; 64 rows of the same 278 -> 177 and 300 -> 195; 945 x 5376 -> 21504 231 -> 217; 1537 x 5376 -> 28672 470 -> 423.
+uint32_t row_tile(uint32_t m, uint32_t nt)
+{
+    constexpr struct {
+        uint32_t rows, time;
+    } kTiles[] = {{256, 100}, {192, 86}, {128, 68}, {64, 55}};
+    const uint64_t cus = uint64_t(std::max(mh3::host::cu_count(), 1));
+    uint64_t best = ~0ull;
+    uint32_t rows = 256;
+    for (const auto& t : kTiles) {
+        const uint64_t tiles = (uint64_t(m) + t.rows - 1u) / t.rows * nt, cost = (tiles + cus - 1u) / cus * t.time;
+        if (cost < best)
+            best = cost, rows = t.rows;
+    }
+    return rows;
+}
+
+// The launch with row tiles of BM rows.
+template <int BM, int MODE, int EPI>
+int launch_tile(const MH3GemmArgs* a, const void* x, const void* w, const float* scale, const float* xscale,
+                uint16_t* out, const mh3::GemmGate& gg, uint32_t nt, mh3_stream_t stream)
+{
+    using namespace mh3;
+    constexpr int WM = kGemmWM, WN = kGemmWN;
+    const auto kernel = &gemm_kernel<BM, WM, WN, MODE, EPI>;
+    constexpr size_t kLds = GemmRing<BM, MODE == kW8A16>::kBytes;
+    if (const hipError_t e = host::allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds); e != hipSuccess)
+        return host::hip_error(e);
+    const uint32_t mt = (a->m + uint32_t(BM) - 1u) / uint32_t(BM);
+    hipLaunchKernelGGL(kernel, dim3(mt * nt), dim3(WM * WN * 64), kLds, static_cast<hipStream_t>(stream), x, w, scale,
+                       xscale, out, a->m, a->n, a->k, mt, nt, gg);
+    return host::check_launch();
+}
 
 // Shared checks and launch of the three forms and three epilogues.
 template <int MODE, int EPI>
@@ -521,17 +600,19 @@ int launch_gemm(const MH3GemmArgs* a, const void* x, const void* w, const float*
          (host::overlaps(out, out_bytes, gg.gate, (uint64_t(gg.n_sets) - 1u) * gg.gate_stride * 4u + a->n * 4ull) ||
           host::overlaps(out, out_bytes, gg.set_of_row, gg.set_of_row ? uint64_t(a->m) : 0u))))
         return MH3_ERR_PARAM;
-    constexpr int WM = kGemmWM, WN = kGemmWN;
-    const void* kernel = reinterpret_cast<const void*>(&gemm_kernel<WM, WN, MODE, EPI>);
-    if (const hipError_t e = host::allow_dynamic_lds(kernel, kGemmLds); e != hipSuccess)
-        return host::hip_error(e);
-    const uint32_t mt = (a->m + kBM - 1) / kBM, nt = a->n / kCols;
-    const uint64_t tiles = uint64_t(mt) * nt;
-    if (tiles >= (uint64_t(1) << 31))
+    const uint32_t nt = a->n / kCols;
+    if (uint64_t((a->m + kBM - 1) / kBM) * nt >= (uint64_t(1) << 31))
         return MH3_ERR_SHAPE;
-    hipLaunchKernelGGL((gemm_kernel<WM, WN, MODE, EPI>), dim3(uint32_t(tiles)), dim3(WM * WN * 64), kGemmLds,
-                       static_cast<hipStream_t>(stream), x, w, scale, xscale, out, a->m, a->n, a->k, mt, nt, gg);
-    return host::check_launch();
+    switch (row_tile(a->m, nt)) {
+    case 64:
+        return launch_tile<64, MODE, EPI>(a, x, w, scale, xscale, out, gg, nt, stream);
+    case 128:
+        return launch_tile<128, MODE, EPI>(a, x, w, scale, xscale, out, gg, nt, stream);
+    case 192:
+        return launch_tile<192, MODE, EPI>(a, x, w, scale, xscale, out, gg, nt, stream);
+    default:
+        return launch_tile<256, MODE, EPI>(a, x, w, scale, xscale, out, gg, nt, stream);
+    }
 }
 
 const mh3::GemmGate kNoGate{nullptr, nullptr, 0, 0};

@@ -225,3 +225,43 @@ def test_gemm_i8_768p_every_row(dev):
     want = orc.gemm_i8_swiglu(x[ti].cpu().numpy(), sx[ti].cpu().numpy(), w.cpu().numpy(), sw.cpu().numpy())
     g = bits_to_f64(to_bits(out[ti]))
     assert_close(g, bits_to_f64(want), 1e-2, 1e-4, "int8 fc1 768p")
+
+
+@pytest.mark.parametrize("form", ["w8a16", "bf16", "w8a8"])
+@pytest.mark.parametrize("k", [128, 256, 384, 640])
+def test_gemm_row_tiles(dev, form, k):
+    """Every row tile (64 column tiles on 256 CUs: 1021 rows take 256-row tiles, 763 192, 505 128, 255 and 33 64), its
+    last rows missing, at K-step counts around the LDS rings' depths: every element against float64 products, and the
+    rows of a smaller batch bit-identical to the same rows of the larger one (the row tile changes no sum's order)."""
+    g = torch.Generator(device=dev).manual_seed(k)
+    m_max, n = 1021, 64 * 128
+    xf = torch.randn((m_max, k), generator=g, device=dev).to(torch.bfloat16)
+    wf = (0.02 * torch.randn((2 * n, k), generator=g, device=dev)).to(torch.bfloat16)
+    x, xs = mh.quant_rows_i8(xf) if form == "w8a8" else (xf, None)
+    w, ws = (wf, None) if form == "bf16" else mh.quant_rows_i8(wf)
+    gate = torch.randn(2 * n, generator=g, device=dev)
+    res0 = torch.randn((m_max, 2 * n), generator=g, device=dev)
+
+    def run(m):
+        xm, sm = x[:m], None if xs is None else xs[:m].contiguous()
+        if form == "w8a16":
+            f = mh.gemm_w8a16_swiglu(xm, w, ws, out=nan_filled((m, n), dev))
+        elif form == "bf16":
+            f = mh.gemm_bf16_swiglu(xm, w, out=nan_filled((m, n), dev))
+        else:
+            f = mh.gemm_i8_swiglu(xm, sm, w, ws, out=nan_filled((m, n), dev))
+        y = mh.gemm(xm, w, x_scale=sm, w_scale=ws, out=nan_filled((m, 2 * n), dev))
+        r = mh.gemm_gate_add(xm, w, res0[:m].to(torch.bfloat16), gate, x_scale=sm, w_scale=ws)
+        r32 = mh.gemm_gate_add(xm, w, res0[:m].clone(), gate, x_scale=sm, w_scale=ws)
+        return f, y, r, r32
+
+    full = run(m_max)
+    check_gemm_full(full[0], x, w, f"{form} fc1", x_scale=xs, w_scale=ws, epi="swiglu")
+    check_gemm_full(full[1], x, w, f"{form} store", x_scale=xs, w_scale=ws)
+    check_gemm_full(full[2], x, w, f"{form} gate_add", x_scale=xs, w_scale=ws, epi="gate_add",
+                    residual0=res0.to(torch.bfloat16), gate=gate)
+    check_gemm_full(full[3], x, w, f"{form} gate_add_f32", x_scale=xs, w_scale=ws, epi="gate_add", residual0=res0,
+                    gate=gate)
+    for m in (763, 505, 255, 33):
+        for name, a, b in zip(("fc1", "store", "gate_add", "gate_add_f32"), run(m), full):
+            assert torch.equal(a, b[:m]), f"{form} {name} k {k} m {m}"

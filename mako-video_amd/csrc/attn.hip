@@ -18,8 +18,9 @@
 // - The output is also transposed, O^T += V^T P^T. P^T is the B operand as the score accumulator leaves it in
 //   registers; the contraction order over keys is free, so the V^T fragment's key positions follow it: position p of
 //   16-key chunk c is key 32 (c / 2) + 16 (c % 2) + 8 (p % 8 / 4) + 4 (p / 8) + p % 4.
-// - K and V tiles (64 rows each, 32 KB) go from global memory straight into LDS (buffer_load ... lds), one tile
-//   ahead of the MFMAs when two stages fit. Each lane fetches whichever source chunk its LDS slot holds, so the
+// - K and V tiles (64 rows each, 32 KB) go from global memory straight into LDS (buffer_load ... lds), one stage: four
+//   workgroups share a CU, and one's loads arrive while the others compute. (Two stages, and the next tile's K during
+//   P V with its V during the scores, measured slower.) Each lane fetches whichever source chunk its LDS slot holds, so the
 //   layouts are free, with one constraint from the address unit: the four lanes of a quad must fetch one aligned
 //   64-byte piece (a quad spread over four rows is four accesses, and held the K/V stream to about 16 bytes a clock a
 //   CU). K is 256-byte rows whose 16-byte chunks are XOR-swizzled by the row (operand reads of 16 rows hit distinct
@@ -36,6 +37,12 @@
 //   lists instead: they start in step (the whole first round at once, and the next rounds nearly so), and tiles in
 //   step share their K/V tiles by walking together. 5 heads at 768p: 7.37-7.40 ms against 7.96-7.98 rotated from
 //   the first tile and 7.73-7.75 never rotated; 40 heads: 54.0-54.4 against 54.2-54.6 (68.1 never rotated).
+// - A grid that is not a multiple of 4 in every direction leaves cubes at its edge with few tokens (16 of 64 slots in a
+//   one-frame image, 32 or less in 37% of the cubes of 37 x 17 x 30). The PACK kernel walks a list's whole cubes first
+//   and then its other cubes' tokens in groups of 16, four groups of any cubes to a key tile, so key tiles are full but
+//   for the last; queries are numbered by token too, so a wave that none falls to only loads. 37 x 17 x 30, 56 heads, ratio
+//   0.1: 3.35 -> 2.22 ms, every cube selected 22.3 -> 16.3 (together with the loads' addresses worked out without
+//   branches); 1 x 43 x 84, 40 heads, ratio 0.5: 3.64 -> 1.05.
 // - Softmax in base 2 with the scale folded into the exponent. A query's running maximum moves only when a tile
 //   raises it by more than 8 (in log2 units): P stays below 2^8, and most tiles skip the rescale of O.
 #include "mh3_common.hpp"
@@ -49,12 +56,11 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr uint32_t kAttnThreads = 128;
-
 constexpr bool kAttnSweep = true; // rotate each cube tile's pass list so an XCD's resident tiles sweep the keys together
 constexpr uint32_t kAttnInStep = 4; // rounds of an XCD's cube tiles that walk their lists unrotated (1, 2, 8: slower;
                                     // 3, 5, 6: within 1%)
-constexpr int kAttnStages = 1;    // K/V stages in LDS (2 overlaps a tile's loads with the previous tile's MFMAs but
-                                  // halves the workgroups a CU holds; one stage and two waves a SIMD measured faster)
+constexpr uint32_t kSegEntries = 512;             // pass-list entries a segment holds (PACK)
+constexpr uint32_t kSegWords = 3u * kSegEntries;  // a whole cube takes one word, another at most 3 groups
 constexpr uint32_t kNoTile = 0xffffffffu;
 
 struct AttnParams {
@@ -132,6 +138,24 @@ __device__ __forceinline__ uint64_t slot_row(const AttnParams& p, const Tile& r,
     return r.base + (r.kind == 1 ? uint64_t(grid_offset(p, l)) : uint64_t(l));
 }
 
+// The tokens of a cube tile (none of another), and the row, from the tile's base, of its i-th token counted without the
+// padding (i < 64). A division by 1 .. 4 is a multiplication by 128 / d rounded up and a shift (exact for i < 64).
+__device__ __forceinline__ uint32_t tile_tokens(const Tile& r) { return r.lim_t * r.lim_y * r.lim_x; }
+__device__ __forceinline__ uint32_t small_recip(uint32_t d) { return d == 1u ? 128u : d == 2u ? 64u : d == 3u ? 43u : 32u; }
+struct TokenRows {
+    uint32_t mx, nx, my, ny, sy, st; // reciprocals and limits of x and y; rows a step in y and t takes
+    __device__ __forceinline__ TokenRows(const AttnParams& p, const Tile& r)
+        : mx(small_recip(r.lim_x)), nx(r.lim_x), my(small_recip(r.lim_y)), ny(r.lim_y), sy(r.kind == 1 ? p.gw : 4u),
+          st(r.kind == 1 ? p.gh * p.gw : 16u)
+    {
+    }
+    __device__ __forceinline__ uint32_t operator()(uint32_t i) const
+    {
+        const uint32_t a = (i * mx) >> 7, dt = (a * my) >> 7;
+        return dt * st + (a - dt * ny) * sy + (i - a * nx);
+    }
+};
+
 __device__ __forceinline__ uint4 load16(const uint16_t* p)
 {
     return *reinterpret_cast<const uint4*>(p);
@@ -158,6 +182,7 @@ __device__ __forceinline__ void lds_barrier()
 }
 
 constexpr uint32_t kStageBytes = 32768; // K 16 KB, then V 16 KB
+constexpr uint32_t kSegBytes = 4u * (kSegWords + 2u * kSegEntries / 64u);
 constexpr uint32_t kPastEnd = 0x80000000u; // a buffer offset past num_records: the load reads zeros
 constexpr uint32_t kRecords = 0x7fffffffu;
 
@@ -166,10 +191,10 @@ __device__ __forceinline__ bool tile_full(const Tile& r)
     return r.kind == 0 ? r.lim_t == 64u : (r.kind != 3 && r.lim_t == 4u && r.lim_y == 4u && r.lim_x == 4u);
 }
 
-template <int STAGES>
-__global__ __launch_bounds__(kAttnThreads, STAGES == 2 ? 1 : 2) void attn_sparse_kernel(AttnParams p)
+template <bool PACK>
+__global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams p)
 {
-    extern __shared__ __attribute__((aligned(16))) char lds[]; // STAGES x (K stage, V stage)
+    extern __shared__ __attribute__((aligned(16))) char lds[]; // K, V; with PACK the segment's entries (kSegWords)
 
     const uint32_t tid = threadIdx.x, lane = tid & 63u, n = lane & 31u, hh = lane >> 5;
     // The wave index is uniform: held in a scalar register, the DMA's per-instruction row offsets (soffset) are
@@ -215,7 +240,6 @@ __global__ __launch_bounds__(kAttnThreads, STAGES == 2 ? 1 : 2) void attn_sparse
         list = p.idx + item * p.out_stride;
         n_sel = uint32_t(min(max(p.cnt[item], 0), int32_t(p.out_stride)));
     }
-    const uint32_t n_tiles = n_sel + p.nd;
     // The pass list is walked from position rot, wrapping round: a workgroup that starts when the XCD's resident ones
     // are a fraction f into their lists starts a fraction f into its own, so the resident tiles sweep the key cubes
     // together and a K/V tile fetched for one is still in that XCD's L2 when the others that selected it reach it.
@@ -223,14 +247,12 @@ __global__ __launch_bounds__(kAttnThreads, STAGES == 2 ? 1 : 2) void attn_sparse
     // The order only changes the softmax's summation order.
     const bool rotated = !dense_q && p.sweep && rank >= kAttnInStep * p.sweep;
     const uint32_t rot = rotated ? uint32_t(uint64_t(rank % p.sweep) * n_sel / p.sweep) : 0u;
-    auto key_tile = [&](uint32_t e) -> uint32_t {
-        if (e >= n_sel)
-            return e - n_sel;
+    auto key_cube = [&](uint32_t e) -> uint32_t { // entry e < n_sel: its key cube, or kNoTile
         if (dense_q)
-            return p.nd + e;
+            return e;
         const uint32_t ee = e + rot < n_sel ? e + rot : e + rot - n_sel;
         const int32_t j = list[ee];
-        return j >= 0 && uint32_t(j) < p.cubes ? p.nd + uint32_t(j) : kNoTile;
+        return j >= 0 && uint32_t(j) < p.cubes ? uint32_t(j) : kNoTile;
     };
 
     // DMA source offsets of this wave's 8 K and 8 V instructions. Instruction i = 8 wave + u of the workgroup's 16
@@ -247,42 +269,83 @@ __global__ __launch_bounds__(kAttnThreads, STAGES == 2 ? 1 : 2) void attn_sparse
     // term of i alone (soffset).
     const uint32_t rs2 = uint32_t(p.row_stride) * 2u, gw_rs2 = p.gw * rs2;
     const uint32_t k_row = lane >> 4, k_pos = lane & 15u, v_key = (lane >> 2) & 3u;
-    const uint32_t v_lane_off = v_key * rs2 + 16u * (4u * (lane >> 4) + (lane & 3u));
-    // Starts tile t's loads into stage st; returns its key mask (bit l: slot l is a token).
-    auto dma_tile = [&](uint32_t t, uint32_t st) -> uint64_t {
-        const Tile tl = make_tile(p, t);
-        const uint64_t row_bytes = (tl.kind == 3 ? 0ull : tl.base) * p.row_stride * 2ull;
-        const __amdgpu_buffer_rsrc_t rk =
-            __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(const_cast<uint16_t*>(kh)) + row_bytes, 0,
-                                              int(kRecords), kRsrcFlags);
-        const __amdgpu_buffer_rsrc_t rv =
-            __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<char*>(const_cast<uint16_t*>(vh)) + row_bytes, 0,
-                                              int(kRecords), kRsrcFlags);
-        char* ks = lds + st * kStageBytes;
-        char* vs = ks + 16384;
-        const bool full = tile_full(tl), grid = tl.kind == 1;
+    const uint32_t v_chunk = 16u * (4u * (lane >> 4) + (lane & 3u)), v_off = v_key * rs2 + v_chunk;
+    uint32_t k_chunk[4]; // K chunk (L % 16) ^ (r % 16), r % 16 = 4 (i % 4) + L / 16
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const uint32_t i = 8u * wave + uint32_t(u);
-            const uint32_t s_i = grid ? ((i >> 2) * p.gh + (i & 3u)) * gw_rs2 : 4u * i * rs2; // slot 4 i's row
-            // K chunk (L % 16) ^ (r % 16), r % 16 = 4 (i % 4) + L / 16
-            uint32_t ko = k_row * rs2 + 16u * (k_pos ^ (4u * (i & 3u) + k_row)), vo = v_lane_off;
-            if (!full) {
-                ko = slot_token(tl, 4u * i + k_row) ? ko : kPastEnd;
-                vo = slot_token(tl, 4u * i + v_key) ? vo : kPastEnd;
+    for (uint32_t u = 0; u < 4; ++u)
+        k_chunk[u] = 16u * (k_pos ^ (4u * u + k_row));
+    auto rsrc_of = [&](const uint16_t* head, uint64_t row) {
+        return __builtin_amdgcn_make_buffer_rsrc(
+            reinterpret_cast<char*>(const_cast<uint16_t*>(head)) + row * p.row_stride * 2ull, 0, int(kRecords), kRsrcFlags);
+    };
+    // Starts tile t's loads; returns its key mask (bit l: slot l is a token). A cube here is whole (a call whose grid
+    // has padding takes the kernel with PACK, which gives it only whole cubes); a dense run may end early.
+    auto dma_tile = [&](uint32_t t) -> uint64_t {
+        const Tile tl = make_tile(p, t);
+        const uint32_t live = tl.kind == 0 ? tl.lim_t : tl.kind == 3 ? 0u : 64u;
+        const __amdgpu_buffer_rsrc_t rk = rsrc_of(kh, tl.base), rv = rsrc_of(vh, tl.base);
+        // Slot 4 i's row, i = 8 wave + u, from the tile's base, in bytes.
+        const uint32_t st = tl.kind == 1 ? p.gh * gw_rs2 : 16u * rs2, sy = tl.kind == 1 ? gw_rs2 : 4u * rs2;
+        const uint32_t s0 = 2u * wave * st;
+        char* const dst = lds + 8192u * wave;
+        if (live == 64u) {
+#pragma unroll
+            for (uint32_t u = 0; u < 8; ++u) {
+                const int so = int(s0 + (u >> 2) * st + (u & 3u) * sy);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)(dst + 1024u * u), 16,
+                                                         k_row * rs2 + k_chunk[u & 3u], so, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)(dst + 16384u + 1024u * u), 16, v_off, so, 0, 0);
             }
-            const int so = int(__builtin_amdgcn_readfirstlane(s_i));
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)(ks + 1024u * i), 16, ko, so, 0, 0);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)(vs + 1024u * i), 16, vo, so, 0, 0);
+            return ~0ull;
         }
-        return full ? ~0ull : __ballot(slot_token(tl, lane));
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) {
+            const uint32_t slot = 32u * wave + 4u * u, ko = k_row * rs2 + k_chunk[u & 3u];
+            const int so = int(s0 + (u >> 2) * st + (u & 3u) * sy);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)(dst + 1024u * u), 16,
+                                                     slot + k_row < live ? ko : kPastEnd, so, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)(dst + 16384u + 1024u * u), 16,
+                                                     slot + v_key < live ? v_off : kPastEnd, so, 0, 0);
+        }
+        return (1ull << live) - 1ull;
+    };
+    // PACK: a tile of `groups` (up to four) groups of 16 tokens, each of some cube at the grid's edge: lane g (of each
+    // four) holds group g's word, the cube in its low 30 bits and the group's number in it above. Each wave loads two of
+    // the groups; a lane works out its own key's row.
+    auto dma_packed = [&](uint32_t word, uint32_t groups) -> uint64_t {
+#pragma unroll
+        for (uint32_t gg = 0; gg < 2; ++gg) {
+            const uint32_t g = 2u * wave + gg, w = __builtin_amdgcn_readlane(word, gg + 2u * wave);
+            const Tile tl = make_tile(p, p.nd + (w & 0x3fffffffu));
+            const uint32_t first = 16u * (w >> 30), tokens = g < groups ? tile_tokens(tl) : 0u;
+            const TokenRows row(p, tl);
+            const __amdgpu_buffer_rsrc_t rk = rsrc_of(kh, tl.base), rv = rsrc_of(vh, tl.base);
+            char* const dst = lds + 4096u * g;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const uint32_t kk = first + 4u * u + k_row, vk = first + 4u * u + v_key;
+                const uint32_t ko = row(kk) * rs2 + k_chunk[u], vo = row(vk) * rs2 + v_chunk;
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rk, (lds_ptr_t)(dst + 1024u * u), 16,
+                                                         kk < tokens ? ko : kPastEnd, 0, 0, 0);
+                __builtin_amdgcn_raw_ptr_buffer_load_lds(rv, (lds_ptr_t)(dst + 16384u + 1024u * u), 16,
+                                                         vk < tokens ? vo : kPastEnd, 0, 0, 0);
+            }
+        }
+        // Slot l is token l % 16 of group l / 16.
+        const uint32_t w = uint32_t(__builtin_amdgcn_ds_bpermute(int(lane >> 4) * 4, int(word)));
+        const Tile tl = make_tile(p, p.nd + (w & 0x3fffffffu));
+        return __ballot((lane >> 4) < groups && 16u * (w >> 30) + (lane & 15u) < tile_tokens(tl));
     };
 
     // This wave's 32 queries as the B operand of S^T = K Q^T: lane (n, hh) holds d 16 dc + 8 hh .. + 7 of query n.
     const Tile qtile = make_tile(p, qt);
+    // Query i of a tile is its slot i; with PACK the i-th token of a cube tile, so that a wave none of them falls to
+    // (a cube of up to 32 tokens) only loads.
     const uint32_t qslot = 32u * wave + n;
-    const bool q_token = slot_token(qtile, qslot);
-    const uint64_t qrow = slot_row(p, qtile, qslot);
+    const bool by_token = PACK && (qtile.kind == 1 || qtile.kind == 2);
+    const bool q_token = by_token ? qslot < tile_tokens(qtile) : slot_token(qtile, qslot);
+    const uint64_t qrow = by_token ? qtile.base + TokenRows(p, qtile)(qslot) : slot_row(p, qtile, qslot);
+    const bool idle = by_token && 32u * wave >= tile_tokens(qtile);
     bf16x8_t qf[8];
 #pragma unroll
     for (int dc = 0; dc < 8; ++dc) {
@@ -305,16 +368,10 @@ __global__ __launch_bounds__(kAttnThreads, STAGES == 2 ? 1 : 2) void attn_sparse
     const uint32_t L = lane & 15u, grp = lane >> 4;
     const uint32_t v_lane = 1024u * (grp >> 1) + 32u * (grp & 1u) + 64u * (L >> 2) + 8u * (L & 3u);
 
-    uint64_t mask = n_tiles ? dma_tile(key_tile(0), 0) : 0ull;
-    for (uint32_t e = 0; e < n_tiles; ++e) {
-        const uint32_t st = STAGES == 2 ? (e & 1u) : 0u;
-        wait_vm0();
-        lds_barrier(); // tile e is in LDS for every wave; every wave is done with tile e - 1
-        uint64_t mask_next = 0;
-        if (STAGES == 2 && e + 1 < n_tiles)
-            mask_next = dma_tile(key_tile(e + 1), st ^ 1u);
-        const char* ks = lds + st * kStageBytes;
-        const char* vs = lds + st * kStageBytes + 16384u + v_lane;
+    // One tile: its scores, their softmax, and its part of the output.
+    auto attend = [&](uint64_t mask) {
+        const char* ks = lds;
+        const char* vs = lds + 16384u + v_lane;
 
         // S^T: lane (n, hh), element i of block b is key 32 b + 8 (i / 4) + 4 hh + i % 4 of query n.
         floatx16 s[2];
@@ -389,25 +446,116 @@ __global__ __launch_bounds__(kAttnThreads, STAGES == 2 ? 1 : 2) void attn_sparse
                 o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pf, o[db], 0, 0, 0);
             }
         }
-        if (STAGES == 1) {
-            lds_barrier(); // every wave is done with the stage before it is refilled
-            if (e + 1 < n_tiles)
-                mask_next = dma_tile(key_tile(e + 1), 0);
+    };
+    // `count` tiles: entry(v) names tile v, fetched while the tile before it is in flight; load(v, entry) starts its
+    // loads and returns its key mask.
+    auto walk = [&](uint32_t count, auto entry, auto load) {
+        uint32_t next = count ? entry(0u) : 0u;
+        for (uint32_t v = 0; v < count; ++v) {
+            const uint64_t mask = load(v, next);
+            if (v + 1u < count)
+                next = entry(v + 1u);
+            wait_vm0();
+            lds_barrier(); // tile v is in LDS for every wave
+            if (!PACK || !idle)
+                attend(mask);
+            lds_barrier(); // every wave is done with it before it is overwritten
         }
-        mask = mask_next;
+    };
+    if constexpr (!PACK) {
+        walk(
+            n_sel + p.nd,
+            [&](uint32_t e) {
+                const uint32_t c = e < n_sel ? key_cube(e) : 0u;
+                return e >= n_sel ? e - n_sel : c == kNoTile ? kNoTile : p.nd + c;
+            },
+            [&](uint32_t, uint32_t tile) { return dma_tile(tile); });
+    } else {
+        // The entries a segment at a time: its whole cubes from the front of seg[], and the groups of 16 tokens of the
+        // others from the back, each in list order.
+        uint32_t* const seg = reinterpret_cast<uint32_t*>(lds + kStageBytes);
+        uint32_t* const counts = seg + kSegWords; // per 64 entries: whole cubes, groups
+        for (uint32_t s0 = 0;; s0 += kSegEntries) {
+            const uint32_t n_seg = min(kSegEntries, n_sel - min(s0, n_sel)), runs = (n_seg + 63u) / 64u;
+            const bool last = s0 + kSegEntries >= n_sel;
+            uint32_t word[kSegEntries / kAttnThreads], n_groups[kSegEntries / kAttnThreads];
+            bool whole[kSegEntries / kAttnThreads];
+#pragma unroll
+            for (uint32_t k = 0; k < kSegEntries / kAttnThreads; ++k) {
+                const uint32_t e = kAttnThreads * k + tid;
+                word[k] = e < n_seg ? key_cube(s0 + e) : kNoTile;
+                const Tile tl = make_tile(p, word[k] == kNoTile ? kNoTile : p.nd + word[k]);
+                whole[k] = tile_full(tl);
+                n_groups[k] = whole[k] ? 0u : (tile_tokens(tl) + 15u) / 16u; // 0 .. 3
+                const uint32_t nw = uint32_t(__popcll(__ballot(whole[k])));
+                const uint32_t ng = uint32_t(__popcll(__ballot(n_groups[k] & 1u)) + 2 * __popcll(__ballot(n_groups[k] & 2u)));
+                if (lane == 0 && 2u * k + wave < runs) {
+                    counts[2u * (2u * k + wave)] = nw;
+                    counts[2u * (2u * k + wave) + 1u] = ng;
+                }
+            }
+            lds_barrier();
+            uint32_t n_whole = 0, n_group = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < kSegEntries / kAttnThreads; ++k) {
+                const uint64_t below = lanes_below(int(lane));
+                uint32_t at_w = n_whole, at_g = n_group;
+#pragma unroll
+                for (uint32_t w = 0; w < 2; ++w) {
+                    if (2u * k + w >= runs)
+                        continue;
+                    const uint32_t nw = counts[2u * (2u * k + w)], ng = counts[2u * (2u * k + w) + 1u];
+                    at_w += w < wave ? nw : 0u;
+                    at_g += w < wave ? ng : 0u;
+                    n_whole += nw;
+                    n_group += ng;
+                }
+                at_w += uint32_t(__popcll(__ballot(whole[k]) & below));
+                at_g += uint32_t(__popcll(__ballot(n_groups[k] & 1u) & below) + 2 * __popcll(__ballot(n_groups[k] & 2u) & below));
+                if (whole[k])
+                    seg[at_w] = word[k];
+                for (uint32_t g = 0; g < n_groups[k]; ++g)
+                    seg[kSegWords - 1u - (at_g + g)] = word[k] | g << 30;
+            }
+            lds_barrier();
+            n_whole = __builtin_amdgcn_readfirstlane(n_whole);
+            n_group = __builtin_amdgcn_readfirstlane(n_group);
+            const uint32_t packed = (n_group + 3u) / 4u;
+            walk(
+                n_whole + packed + (last ? p.nd : 0u),
+                [&](uint32_t v) -> uint32_t {
+                    const uint32_t g0 = 4u * (v - n_whole); // of a packed tile: its first group
+                    return seg[v < n_whole              ? v
+                               : v - n_whole < packed ? kSegWords - 1u - min(g0 + (lane & 3u), n_group - 1u)
+                                                      : 0u];
+                },
+                [&](uint32_t v, uint32_t word) {
+                    if (v - n_whole < packed)
+                        return dma_packed(word, min(n_group - 4u * (v - n_whole), 4u));
+                    return dma_tile(v < n_whole ? p.nd + __builtin_amdgcn_readfirstlane(word) : v - n_whole - packed);
+                });
+            if (last)
+                break;
+        }
     }
 
     // Normalize and write the query rows (a gathered cube's padding slots get zeros; other non-tokens nothing).
     const float l_tot = l_run + __shfl_xor(l_run, 32, kWave);
     const float inv = q_token && l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-    if (q_token || qtile.kind == 2) {
+    if (PACK && qtile.kind == 2 && !slot_token(qtile, qslot)) {
+        uint16_t* orow = p.out + hoff + slot_row(p, qtile, qslot) * p.row_stride;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            *reinterpret_cast<uint4*>(orow + 16 * j + 8u * hh) = uint4{0u, 0u, 0u, 0u};
+    }
+    if (q_token || (!PACK && qtile.kind == 2)) {
         uint16_t* orow = p.out + hoff + qrow * p.row_stride;
 #pragma unroll
         for (int db = 0; db < 4; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const uint32_t d0 = 32u * db + 8u * g + 4u * hh;
-                const uint2 w = q_token ? uint2{pack_bf16(o[db][4 * g] * inv, o[db][4 * g + 1] * inv),
+                const uint2 w = PACK || q_token ? uint2{pack_bf16(o[db][4 * g] * inv, o[db][4 * g + 1] * inv),
                                                 pack_bf16(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv)}
                                         : uint2{0u, 0u}; // +0, not the sign of 0 * o
                 *reinterpret_cast<uint2*>(orow + d0) = w;
@@ -500,9 +648,10 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     const float scale = args->scale > 0.0f ? args->scale : 0.08838834764831845f; // 1 / sqrt(128)
     p.scale_log2 = scale * 1.4426950408889634f;
     const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
-    constexpr int kStages = kAttnStages;
-    const void* kern = reinterpret_cast<const void*>(&attn_sparse_kernel<kStages>);
-    const size_t lds = size_t(kStages) * kStageBytes;
+    const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0;
+    const auto kernel = pack ? &attn_sparse_kernel<true> : &attn_sparse_kernel<false>;
+    const void* kern = reinterpret_cast<const void*>(kernel);
+    const size_t lds = kStageBytes + (pack ? kSegBytes : 0u);
     if (const hipError_t e = host::allow_dynamic_lds(kern, lds); e != hipSuccess)
         return host::hip_error(e);
     if (kAttnSweep) {
@@ -513,8 +662,7 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
         // The sweep period: the cube workgroups an XCD holds at once (half or twice that measured slower).
         p.sweep = uint32_t(uint64_t(std::max(per_cu, 1)) * uint32_t(host::cu_count()) / 8u);
     }
-    hipLaunchKernelGGL(attn_sparse_kernel<kStages>, dim3(uint32_t(blocks)), dim3(kAttnThreads), lds,
-                       static_cast<hipStream_t>(stream), p);
+    hipLaunchKernelGGL(kernel, dim3(uint32_t(blocks)), dim3(kAttnThreads), lds, static_cast<hipStream_t>(stream), p);
     return host::check_launch();
 }
 

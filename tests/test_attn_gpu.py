@@ -344,3 +344,47 @@ def test_flash_attn_sparse_heads_over_the_xcds(dev, heads, grid, layout, n_dense
                                        out=nan_filled((heads, rows, 128), dev), order=order)
         ref = attn_sparse_f32(q, k, v, idx, cnt, grid, video, n_dense, layout=layout)
         check_attn_f32(out, ref, f"{heads} heads {grid}")
+
+
+@pytest.mark.parametrize("grid,layout,n_dense,kk", [
+    ((1, 7, 11), orc.CUBES_GRID, 5, 3),            # one frame: 16 tokens a cube and fewer
+    ((2, 6, 9), orc.CUBES_GATHERED, 70, 6),        # 32 a cube; every cube selected
+    ((3, 4, 8), orc.CUBES_GRID, 0, 1),             # 48 a cube, no dense rows
+    ((7, 9, 10), orc.CUBES_GRID, 64, 7),           # 3, 1 and 2 past the last whole cube
+    ((5, 11, 13), orc.CUBES_GATHERED, 130, 9),
+    ((9, 42, 70), orc.CUBES_GRID, 40, 594),        # lists of more entries than a segment, every cube selected
+    ((9, 42, 70), orc.CUBES_GATHERED, 0, 530),
+])
+def test_flash_attn_sparse_packed_edges(dev, grid, layout, n_dense, kk):
+    """Grids with cubes at the edge whose tokens share key tiles: every row against the float32 restatement, into a
+    NaN-filled output, over ascending lists and over shuffled ones with entries outside the cubes and repeated ones;
+    a gathered cube's padding rows zero; an empty list without dense rows zero."""
+    heads, C = 3, orc.cube_count(*grid)
+    video = C * 64 if layout == orc.CUBES_GATHERED else grid[0] * grid[1] * grid[2]
+    rows = 3 + video + n_dense
+    g = torch.Generator(device=dev).manual_seed(C)
+    q, k, v = [torch.randn((heads, rows, 128), generator=g, device=dev).to(torch.bfloat16) for _ in range(3)]
+    rng = np.random.default_rng(C)
+    idx, cnt = orc.cube_topk(rng.standard_normal((heads, C, C)), grid, kk, 1, out_stride=kk + 2)
+    odd = rng.permuted(idx, axis=2)                             # the -1 entries among the others
+    odd[0, :, 0] = C + 5
+    odd[1, :, 0] = odd[1, :, -1] = 0                            # cube 0 twice
+    odd[:, 0] = -1
+    odd[:, 0, :1] = C - 1                                       # only the last cube
+    a = mh.cube_args(heads, grid, layout=layout, row0=3, head_stride=rows * 128, out_stride=kk + 2)
+    for what, idx_n, cnt_n in (("lists", idx, cnt), ("odd lists", odd, np.full_like(cnt, kk + 2))):
+        ti, tc = torch.from_numpy(np.ascontiguousarray(idx_n)).to(dev), torch.from_numpy(cnt_n).to(dev)
+        out = mh.flash_attn_sparse_128(a, q, k, v, ti, tc, dense_row0=3 + video, n_dense=n_dense,
+                                       out=nan_filled((heads, rows, 128), dev))
+        ref = attn_sparse_f32(q, k, v, ti, tc, grid, 3 + video, n_dense, layout=layout, row0=3)
+        check_attn_f32(out, ref, f"{what} {grid}")
+        if layout == orc.CUBES_GATHERED:
+            written = torch.zeros(rows, dtype=torch.bool, device=dev)
+            written[ref[0][0]] = True
+            pad = ~written
+            pad[:3] = False
+            assert bool((out[:, pad].view(torch.int16) == 0).all()), "padding rows"
+    if n_dense == 0:
+        tc = torch.zeros((heads, C), dtype=torch.int32, device=dev)
+        out = mh.flash_attn_sparse_128(a, q, k, v, ti, tc, out=nan_filled((heads, rows, 128), dev))
+        assert bool((out[:, ref[0][0]] == 0).all()), "empty lists"

@@ -42,7 +42,8 @@
 //   and then its other cubes' tokens in groups of 16, four groups of any cubes to a key tile, so key tiles are full but
 //   for the last; queries are numbered by token too, so a wave that none falls to only loads. 37 x 17 x 30, 56 heads, ratio
 //   0.1: 3.35 -> 2.22 ms, every cube selected 22.3 -> 16.3 (together with the loads' addresses worked out without
-//   branches); 1 x 43 x 84, 40 heads, ratio 0.5: 3.64 -> 1.05.
+//   branches); 1 x 43 x 84, 40 heads, ratio 0.5: 3.64 -> 1.05. Fragment reads ahead and the exponentials between the
+//   P V MFMAs then took these to 2.07, 15.5 and 0.93.
 // - Softmax in base 2 with the scale folded into the exponent. A query's running maximum moves only when a tile
 //   raises it by more than 8 (in log2 units): P stays below 2^8, and most tiles skip the rescale of O.
 #include "mh3_common.hpp"
@@ -191,7 +192,8 @@ __device__ __forceinline__ bool tile_full(const Tile& r)
     return r.kind == 0 ? r.lim_t == 64u : (r.kind != 3 && r.lim_t == 4u && r.lim_y == 4u && r.lim_x == 4u);
 }
 
-template <bool PACK>
+// kAhead: how many fragments are read ahead of their MFMAs (stream_bound says which of the two a call takes).
+template <bool PACK, int kAhead>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams p)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[]; // K, V; with PACK the segment's entries (kSegWords)
@@ -372,30 +374,51 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
     auto attend = [&](uint64_t mask) {
         const char* ks = lds;
         const char* vs = lds + 16384u + v_lane;
+        auto read_k = [&](int j) { // key block j % 2, d chunk j / 2
+            return *reinterpret_cast<const bf16x8_t*>(ks + 8192u * (j & 1) + (k_lane ^ (32u * (j >> 1))));
+        };
+        auto read_v = [&](int j) { // 16-key chunk j / 4, d block j % 4: two transposed reads (positions 0-3, 4-7)
+            const uint32_t off = 4096u * (j >> 2) + 256u * (j & 3);
+            const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (v4i16 __attribute__((address_space(3)))*)(const_cast<char*>(vs) + off));
+            const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                (v4i16 __attribute__((address_space(3)))*)(const_cast<char*>(vs) + off + 2048u));
+            return __builtin_bit_cast(bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+        };
 
-        // S^T: lane (n, hh), element i of block b is key 32 b + 8 (i / 4) + 4 hh + i % 4 of query n.
+        // S^T: lane (n, hh), element i of block b is key 32 b + 8 (i / 4) + 4 hh + i % 4 of query n. The fragment reads
+        // go kAhead MFMAs ahead, held in that order (left to itself the compiler reads each right before its MFMA).
         floatx16 s[2];
+        bf16x8_t frag[kAhead];
 #pragma unroll
-        for (int b = 0; b < 2; ++b) {
+        for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int i = 0; i < 16; ++i)
                 s[b][i] = 0.0f;
 #pragma unroll
-            for (int dc = 0; dc < 8; ++dc) {
-                const bf16x8_t a = *reinterpret_cast<const bf16x8_t*>(ks + 8192u * b + (k_lane ^ (32u * dc)));
-                s[b] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, qf[dc], s[b], 0, 0, 0);
-            }
+        for (int j = 0; j < kAhead; ++j)
+            frag[j] = read_k(j);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            __builtin_amdgcn_sched_barrier(0);
+            s[j & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[j % kAhead], qf[j >> 1], s[j & 1], 0, 0, 0);
+            if (j + kAhead < 16)
+                frag[j % kAhead] = read_k(j + kAhead);
         }
+        __builtin_amdgcn_sched_barrier(0);
         // Online softmax in base 2: padding keys score -inf; the maximum moves only when it rises by more than 8.
         float mt = -__builtin_inff();
         if (mask != ~0ull) {
+            // Kept a branch: left to itself the compiler computes all 32 selects for every tile (100 instructions
+            // beside the softmax's 130).
+            asm volatile("" ::: "memory");
 #pragma unroll
-            for (int b = 0; b < 2; ++b)
+            for (int b = 0; b < 2; ++b) {
+                const uint32_t live = uint32_t(mask >> (32 * b)) >> (4u * hh); // bit 8 (i / 4) + i % 4: element i
 #pragma unroll
-                for (int i = 0; i < 16; ++i) {
-                    const uint32_t key = 32u * b + 8u * (i >> 2) + 4u * hh + (i & 3);
-                    s[b][i] = (mask >> key) & 1ull ? s[b][i] : -__builtin_inff();
-                }
+                for (int i = 0; i < 16; ++i)
+                    s[b][i] = live & (1u << (8 * (i >> 2) + (i & 3))) ? s[b][i] : -__builtin_inff();
+            }
         }
 #pragma unroll
         for (int b = 0; b < 2; ++b)
@@ -415,37 +438,42 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
                     o[b][i] *= alpha;
         }
         const float m_ref = m_run == -__builtin_inff() ? 0.0f : m_run;
+        // O^T (d 32 db + 8 (i / 4) + 4 hh + i % 4 of query n) += V^T P^T; P^T chunk c is elements 8 (c % 2) .. + 7 of
+        // block c / 2. V's first fragments arrive during the first chunk's exponentials, and each later chunk's
+        // exponentials go between the MFMAs of the chunk before it.
+#pragma unroll
+        for (int j = 0; j < kAhead; ++j)
+            frag[j] = read_v(j);
+        __builtin_amdgcn_sched_barrier(0);
         float ps = 0.0f;
-        uint32_t pw[2][8];
+        uint32_t pw[2][4];
+        auto exp_pair = [&](int c, int e) { // elements 2 e and 2 e + 1 of chunk c
+            const int b = c >> 1, i = 8 * (c & 1) + 2 * e;
+            const float p0 = __builtin_amdgcn_exp2f(fmaf(s[b][i], p.scale_log2, -m_ref));
+            const float p1 = __builtin_amdgcn_exp2f(fmaf(s[b][i + 1], p.scale_log2, -m_ref));
+            ps += p0 + p1;
+            pw[c & 1][e] = pack_bf16(p0, p1);
+        };
 #pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-            for (int i = 0; i < 16; i += 2) {
-                const float p0 = __builtin_amdgcn_exp2f(fmaf(s[b][i], p.scale_log2, -m_ref));
-                const float p1 = __builtin_amdgcn_exp2f(fmaf(s[b][i + 1], p.scale_log2, -m_ref));
-                ps += p0 + p1;
-                pw[b][i >> 1] = pack_bf16(p0, p1);
-            }
-        l_run += ps;
-        // O^T (d 32 db + 8 (i / 4) + 4 hh + i % 4 of query n) += V^T P^T; P^T chunk c = 2 b + g is accumulator
-        // elements 8 g .. + 7 of block b; its V^T fragment is two transposed reads (positions 0-3, 4-7 of the half).
+        for (int e = 0; e < 4; ++e)
+            exp_pair(0, e);
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
-            const int b = c >> 1, g = c & 1;
-            const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, uint4{pw[b][4 * g], pw[b][4 * g + 1], pw[b][4 * g + 2],
-                                                                   pw[b][4 * g + 3]});
+            const uint32_t* w = pw[c & 1];
+            const bf16x8_t pf = __builtin_bit_cast(bf16x8_t, uint4{w[0], w[1], w[2], w[3]});
 #pragma unroll
             for (int db = 0; db < 4; ++db) {
-                const uint32_t off = 1024u * (8u * b + 4u * g) + 256u * db;
-                const v4i16 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4i16 __attribute__((address_space(3)))*)(
-                    const_cast<char*>(vs) + off));
-                const v4i16 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((v4i16 __attribute__((address_space(3)))*)(
-                    const_cast<char*>(vs) + off + 2048u));
-                const bf16x8_t a = __builtin_bit_cast(
-                    bf16x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, pf, o[db], 0, 0, 0);
+                const int j = 4 * c + db;
+                __builtin_amdgcn_sched_barrier(0);
+                o[db] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(frag[j % kAhead], pf, o[db], 0, 0, 0);
+                if (j + kAhead < 16)
+                    frag[j % kAhead] = read_v(j + kAhead);
+                if (c < 3)
+                    exp_pair(c + 1, db);
             }
         }
+        __builtin_amdgcn_sched_barrier(0);
+        l_run += ps;
     };
     // `count` tiles: entry(v) names tile v, fetched while the tile before it is in flight; load(v, entry) starts its
     // loads and returns its key mask.
@@ -582,6 +610,18 @@ uint32_t share_of(uint32_t heads, uint64_t bytes)
     return share;
 }
 
+// Whether the call waits for the K/V stream past L2 rather than for its own work: a head's K and V (`bytes`) many times
+// an XCD's 4 MB of L2, and lists of so few of its cubes that the tiles on an XCD seldom want the same one at once. The
+// time is then the bytes past L2 over some 7.4 TB/s, whatever a tile's own work takes, and a steadier pace, which
+// keeps the tiles' sweeps together, beats a faster one: reading each fragment right before its MFMA, the hit rate is 41%
+// against 30% (2016 cubes, 40 heads, ratio 0.1: 348 and 418 GB past L2; 48.2 against 54.0 ms, overlapping lists 47.2 and
+// 52.0; 1440 cubes, independent lists 25.1 and 27.1). Elsewhere eight ahead are faster (2016 cubes, 8 heads, ratio 0.3:
+// 33.0 and 31.4 ms; 1024 cubes 12.9 and 12.6; 37 x 17 x 30 dense 16.3 and 15.5).
+bool stream_bound(uint64_t bytes, const mh3::AttnParams& p)
+{
+    return bytes > (40ull << 20) && uint64_t(p.out_stride) * 5u < p.cubes;
+}
+
 // order: null for the plain entry point; `ordered`: the ordered one, which needs it.
 int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, const uint16_t* v, const int32_t* idx,
                 const int32_t* cnt, const int32_t* order, bool ordered, uint16_t* out, mh3_stream_t stream)
@@ -649,7 +689,9 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     p.scale_log2 = scale * 1.4426950408889634f;
     const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
     const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0;
-    const auto kernel = pack ? &attn_sparse_kernel<true> : &attn_sparse_kernel<false>;
+    const auto kernel = pack                                            ? &attn_sparse_kernel<true, 8>
+                        : stream_bound((video + args->n_dense) * 512ull, p) ? &attn_sparse_kernel<false, 1>
+                                                                        : &attn_sparse_kernel<false, 8>;
     const void* kern = reinterpret_cast<const void*>(kernel);
     const size_t lds = kStageBytes + (pack ? kSegBytes : 0u);
     if (const hipError_t e = host::allow_dynamic_lds(kern, lds); e != hipSuccess)

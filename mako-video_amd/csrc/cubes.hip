@@ -224,9 +224,9 @@ constexpr uint32_t kPaddedRow = 64u * (KPL + 4);
 
 // The scores of one key block, stored. A block with a non-finite score (the test is wave-uniform) is scored again by
 // float FMAs (score_block_direct); where `row_flags` is given, rows left with a non-finite score are flagged there.
-// Scores s[r][j] (r < 16, j < cubes) go to `dst` at r * ld + j, or at r * ld + pad_word<32>(j) when PAD (rows past
-// the last query cube skipped).
-template <bool PAD>
+// Scores s[r][j] (r < 16, j < cubes) go to `dst` at r * ld + j, or with KPL at r * ld + pad_word<KPL>(j) (rows past the
+// last query cube skipped).
+template <int KPL>
 __device__ __forceinline__ void store_block(const CubeGeo& g, const float* __restrict__ qh,
                                             const float* __restrict__ kh, uint32_t i0, uint32_t b, floatx4 acc,
                                             float* dst, uint64_t ld, uint32_t* row_flags)
@@ -247,7 +247,7 @@ __device__ __forceinline__ void store_block(const CubeGeo& g, const float* __res
     for (int v = 0; v < 4; ++v) {
         const uint32_t r = (lane >> 4) * 4u + uint32_t(v);
         if (j < g.cubes && i0 + r < g.cubes)
-            dst[r * ld + (PAD ? pad_word<32>(j) : j)] = acc[v] * kScoreScale;
+            dst[r * ld + (KPL ? pad_word<(KPL ? KPL : 1)>(j) : j)] = acc[v] * kScoreScale;
     }
 }
 
@@ -272,7 +272,7 @@ __device__ __forceinline__ void score_rows(const CubeGeo& g, const float* __rest
         split_exchange(kr, ks);
         if (b + waves < kblocks)
             load_raw(kh, (b + waves) * 16u, g.cubes, kr);
-        store_block<false>(g, qh, kh, i0, b, score_block(qs, ks), dst, ld, nullptr);
+        store_block<0>(g, qh, kh, i0, b, score_block(qs, ks), dst, ld, nullptr);
     }
 }
 
@@ -313,6 +313,7 @@ __device__ __forceinline__ void load_split(const uint4* __restrict__ base, uint3
 // cube_select's scoring: as score_rows, with the key blocks' operands from cube_split_kernel (`ksh`: the head's
 // blocks) and the scores into the padded LDS tile, rows with a non-finite score flagged in `row_flags`. One block in
 // flight a wave: 0.525-0.532 ms at 768p against 0.535-0.551 ms for two (registers spilled) and 1.14 ms for three.
+template <int KPL>
 __device__ __forceinline__ void score_rows_split(const CubeGeo& g, const float* __restrict__ qh,
                                                  const float* __restrict__ kh, const uint4* __restrict__ ksh,
                                                  uint32_t i0, float* dst, uint64_t ld, uint32_t wave, uint32_t waves,
@@ -332,7 +333,7 @@ __device__ __forceinline__ void score_rows_split(const CubeGeo& g, const float* 
         const floatx4 acc = score_block(qs, kr);
         if (b + waves < kblocks)
             load_split(ksh, b + waves, kr);
-        store_block<true>(g, qh, kh, i0, b, acc, dst, ld, row_flags);
+        store_block<KPL>(g, qh, kh, i0, b, acc, dst, ld, row_flags);
     }
 }
 
@@ -374,7 +375,7 @@ constexpr uint32_t kHistBins = 128; // lanes 0 .. 31 hold four bins each
 
 // Per-lane bit masks over a lane's KPL cubes.
 template <int KPL>
-using LaneMask = typename std::conditional<KPL == 32, uint32_t, uint64_t>::type;
+using LaneMask = typename std::conditional<KPL <= 32, uint32_t, uint64_t>::type;
 
 // The selection from the threshold's masks, bit m for cube j0 + m of the lane: gt (scores above the k-th largest t)
 // and eq (scores equal to t). The first k - #gt ties in cube order join gt (a prefix sum of per-lane tie counts ranks
@@ -681,10 +682,15 @@ constexpr int kSelectThreads = int(64 * (kSelectScorers + kSelectRankers));
 constexpr uint32_t kSelectRows = 16;
 constexpr uint32_t kSelectMaxCubes = 2048;
 static_assert(2 * kSelectRankers == kSelectRows, "two rows of a tile a ranking wave");
+// KPL: cubes a ranking lane holds of a row, 8, 16 or 32 (the least with room for them all): the ranking's work goes with
+// it, and 400 cubes fill 13 of 64 lanes at 32 but 50 at 8 (56 heads: 87 -> 48 us; 360 cubes 200 -> 152 us with
+// the pool, 896 cubes 359 -> 320).
+template <int KPL>
 constexpr size_t kSelectLds =
-    (size_t(kSelectRows) * kPaddedRow<32> + kSelectRankers * (64u + kHistBins) + kSelectRows) * sizeof(float);
-static_assert(kSelectLds <= 160 * 1024, "the select tile, candidates, histograms and flags fit gfx950's LDS");
+    (size_t(kSelectRows) * kPaddedRow<KPL> + kSelectRankers * (64u + kHistBins) + kSelectRows) * sizeof(float);
+static_assert(kSelectLds<32> <= 160 * 1024, "the select tile, candidates, histograms and flags fit gfx950's LDS");
 
+template <int KPL>
 __global__ __launch_bounds__(kSelectThreads) void cube_select_kernel(CubeGeo g, const float* __restrict__ qc,
                                                                      const float* __restrict__ kc,
                                                                      const uint4* __restrict__ ks, uint32_t k,
@@ -699,13 +705,13 @@ __global__ __launch_bounds__(kSelectThreads) void cube_select_kernel(CubeGeo g, 
     const uint64_t plane = uint64_t(g.cubes) * 128u;
     const uint32_t row_tiles = (g.cubes + kSelectRows - 1u) / kSelectRows, tiles = row_tiles * g.heads;
     uint32_t* row_flags =
-        reinterpret_cast<uint32_t*>(tile + kSelectRows * kPaddedRow<32> + kSelectRankers * (64u + kHistBins));
+        reinterpret_cast<uint32_t*>(tile + kSelectRows * kPaddedRow<KPL> + kSelectRankers * (64u + kHistBins));
     {
         // NaN in each row's slots past the last cube (never scored: the ranking takes them as no score); flags clear.
-        const uint32_t pad = 64u * 32u - g.cubes;
+        const uint32_t pad = 64u * KPL - g.cubes;
         for (uint32_t q = threadIdx.x; q < kSelectRows * pad; q += blockDim.x) {
             const uint32_t r = q / pad, j = g.cubes + (q - r * pad);
-            tile[r * kPaddedRow<32> + pad_word<32>(j)] = __builtin_nanf("");
+            tile[r * kPaddedRow<KPL> + pad_word<KPL>(j)] = __builtin_nanf("");
         }
         if (threadIdx.x < kSelectRows)
             row_flags[threadIdx.x] = 0u;
@@ -715,24 +721,24 @@ __global__ __launch_bounds__(kSelectThreads) void cube_select_kernel(CubeGeo g, 
         const uint32_t kblocks = (g.cubes + 15u) / 16u;
         for (uint32_t t = blockIdx.x; t < tiles; t += gridDim.x) {
             const uint32_t h = t / row_tiles, i0 = (t - h * row_tiles) * kSelectRows;
-            score_rows_split(g, qc + h * plane, kc + h * plane, ks + uint64_t(h) * kblocks * 512u, i0, tile,
-                             kPaddedRow<32>, wave, kSelectScorers, row_flags);
+            score_rows_split<KPL>(g, qc + h * plane, kc + h * plane, ks + uint64_t(h) * kblocks * 512u, i0, tile,
+                             kPaddedRow<KPL>, wave, kSelectScorers, row_flags);
             __syncthreads(); // tile t scored
             __syncthreads(); // the ranking waves hold every row of t: the tile is free
         }
         return;
     }
     const uint32_t r0 = wave - kSelectScorers; // rows r0 and r0 + 8 of each tile
-    uint32_t* cand = reinterpret_cast<uint32_t*>(tile + kSelectRows * kPaddedRow<32>) + r0 * (64u + kHistBins);
-    auto rank_row = [&](uint32_t t, uint32_t r, RowVals<32>& vals, bool finite) {
+    uint32_t* cand = reinterpret_cast<uint32_t*>(tile + kSelectRows * kPaddedRow<KPL>) + r0 * (64u + kHistBins);
+    auto rank_row = [&](uint32_t t, uint32_t r, RowVals<KPL>& vals, bool finite) {
         const uint32_t h = t / row_tiles, i = (t - h * row_tiles) * kSelectRows + r;
         if (i < g.cubes) {
             const uint64_t item = uint64_t(h) * g.cubes + i;
-            topk_vals<32>(vals, finite, g, i, k, local, idx + item * out_stride, out_stride, cnt + item, cand,
+            topk_vals<KPL>(vals, finite, g, i, k, local, idx + item * out_stride, out_stride, cnt + item, cand,
                           cand + 64);
         }
     };
-    RowVals<32> rva, rvb;
+    RowVals<KPL> rva, rvb;
     bool fa = true, fb = true;
     for (uint32_t j = 0;; ++j) {
         const uint32_t t = blockIdx.x + j * gridDim.x;
@@ -743,8 +749,8 @@ __global__ __launch_bounds__(kSelectThreads) void cube_select_kernel(CubeGeo g, 
         if (t >= tiles)
             break;
         __syncthreads(); // tile t scored
-        load_vals<32>(tile + r0 * kPaddedRow<32>, rva);
-        load_vals<32>(tile + (r0 + kSelectRankers) * kPaddedRow<32>, rvb);
+        load_vals<KPL>(tile + r0 * kPaddedRow<KPL>, rva);
+        load_vals<KPL>(tile + (r0 + kSelectRankers) * kPaddedRow<KPL>, rvb);
         fa = __builtin_amdgcn_readfirstlane(row_flags[r0]) == 0u;
         fb = __builtin_amdgcn_readfirstlane(row_flags[r0 + kSelectRankers]) == 0u;
         if ((threadIdx.x & 63u) == 0u)
@@ -1027,7 +1033,10 @@ int mh3_cube_select(const MH3CubeArgs* args, const float* qc, const float* kc, v
     }
     if (g.cubes > kSelectMaxCubes)
         return MH3_ERR_UNSUPPORTED; // more cubes than the LDS tile holds: use cube_scores + cube_topk
-    const int lds_ok = set_lds_limit(reinterpret_cast<const void*>(&cube_select_kernel), kSelectLds);
+    const bool small = g.cubes <= 512u, mid = g.cubes <= 1024u;
+    const auto select = small ? &cube_select_kernel<8> : mid ? &cube_select_kernel<16> : &cube_select_kernel<32>;
+    const size_t lds = small ? kSelectLds<8> : mid ? kSelectLds<16> : kSelectLds<32>;
+    const int lds_ok = set_lds_limit(reinterpret_cast<const void*>(select), lds);
     if (lds_ok != MH3_OK)
         return lds_ok;
     const hipStream_t st = static_cast<hipStream_t>(stream);
@@ -1039,7 +1048,7 @@ int mh3_cube_select(const MH3CubeArgs* args, const float* qc, const float* kc, v
     // Persistent: one workgroup a CU (the tile takes the LDS), at most one a tile.
     const uint32_t tiles = (g.cubes + kSelectRows - 1) / kSelectRows * g.heads;
     const dim3 grid(std::min<uint32_t>(tiles, uint32_t(host::cu_count())));
-    hipLaunchKernelGGL(cube_select_kernel, grid, dim3(kSelectThreads), kSelectLds, st, g, qc, kc, ks, args->k,
+    hipLaunchKernelGGL(select, grid, dim3(kSelectThreads), lds, st, g, qc, kc, ks, args->k,
                        args->local, args->out_stride, idx, cnt);
     return host::check_launch();
 }

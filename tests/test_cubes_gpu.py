@@ -395,3 +395,19 @@ def test_topk_beyond_2048_cubes(dev, local):
     assert (idx.cpu().numpy() == widx).all()
     with pytest.raises(RuntimeError):
         mh.cube_select(a, tq, tk)
+
+
+@pytest.mark.parametrize("cubes", [1, 8, 63, 511, 512, 513, 1024, 1025])
+def test_cube_select_cubes_a_lane(dev, cubes):
+    """Around the counts where a ranking lane holds 8, 16 or 32 cubes of a row: cube_select equal to cube_topk over
+    cube_scores, on random means and on means that tie, with and without local cubes."""
+    heads, grid = 2, (4, 4, 4 * cubes)
+    g = torch.Generator(device=dev).manual_seed(cubes)
+    qc, kc = [torch.randn((heads, cubes, 128), generator=g, device=dev) for _ in range(2)]
+    for name, kk in (("random", kc), ("ties", kc[:, :1].expand(-1, cubes, -1).contiguous())):
+        for k, local in ((1, 1), (max(1, cubes // 3), 3), (cubes, 0)):
+            a = mh.cube_args(heads, grid, k=k, local=local)
+            want = mh.cube_topk(a, mh.cube_scores(a, qc, kk))
+            got = mh.cube_select(a, qc, kk)
+            for x, y in zip(got, want):
+                assert torch.equal(x, y), f"{cubes} cubes, {name}, k {k}, local {local}"

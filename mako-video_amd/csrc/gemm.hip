@@ -10,7 +10,7 @@
 //
 // Design (gfx950, v_mfma_f32_16x16x32_bf16):
 // - A workgroup of 8 wavefronts (2 along rows x 4 along columns) computes a tile of BM = 256 rows (fewer where a call
-//   has too few rows to fill the chip with those: row_tile) x 128 columns, i.e. the 128 gate columns [n0, n0+128) and
+//   has too few rows to fill the chip with those: choose_tile) x 128 columns, i.e. the 128 gate columns [n0, n0+128) and
 //   the 128 up columns [n + n0, n + n0 + 128) of y, so the SwiGLU epilogue has both halves in registers. Each wave
 //   owns BM / 2 rows x (32 gate + 32 up) columns, at 256 rows 8 x 4 MFMA tiles of 16 x 16.
 // - K advances 64 at a time. A (x, bf16) streams from HBM straight into an LDS ring (3 stages) with buffer loads that
@@ -41,16 +41,18 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr uint32_t kBM = 256, kBN = 128, kBK = 64; // kBM: the largest row tile
-// LDS: a ring of A stages (BM rows x 64 k bf16: 8 16-byte chunks a row), then B stages (256 B-rows x 64 k, bf16 or
-// widened to it: 2048 chunks each). 3 A and 2 B stages fill gfx950's 160 KiB at 256 rows. A smaller row tile spends less
+// LDS: a ring of A stages (BM rows x 64 k bf16: 8 16-byte chunks a row), then B stages (2 BN B-rows x 64 k, bf16
+// or widened to it). 3 A and 2 B stages fill gfx950's 160 KiB at 256 rows. A smaller row tile spends less
 // time on a K-step than a load takes to arrive, so where both operands stream into LDS it takes more stages and its
 // loads go out further ahead (128 rows, x [1277][14336] bf16, 21 column tiles: 249 us with 3 and 2, 208 with 4 and 3).
-constexpr uint32_t kBChunks = 2048;
-template <int BM, bool I8>
+// The narrow tile (BN = 32) takes five of each, and with int8 weights three register sets of B: its K-steps are shorter
+// still, and two of its workgroups share a CU.
+template <int BM, int BN, bool I8>
 struct GemmRing {
-    static constexpr uint32_t kAChunks = BM * 8u;
-    static constexpr uint32_t kAStages = BM <= 128 && !I8 ? 4 : 3;
-    static constexpr uint32_t kBStages = I8 ? 2 : BM <= 64 ? 4 : BM <= 128 ? 3 : 2;
+    static constexpr uint32_t kAChunks = BM * 8u, kBChunks = BN * 16u;
+    static constexpr uint32_t kBRegs = BN < 128 ? 3 : 1; // register sets of int8 B
+    static constexpr uint32_t kAStages = BN < 128 ? 5 : BM <= 128 && !I8 ? 4 : 3;
+    static constexpr uint32_t kBStages = I8 ? 2 : BN < 128 ? 5 : BM <= 64 ? 4 : BM <= 128 ? 3 : 2;
     static constexpr size_t kBytes = (size_t(kAStages) * kAChunks + size_t(kBStages) * kBChunks) * 16;
 };
 constexpr uint32_t kBandM = 4; // row tiles an XCD sweeps across all column tiles before moving on
@@ -138,12 +140,12 @@ typedef int int32x4 __attribute__((ext_vector_type(4)));
 
 // The epilogue shared by the GEMM kernels, through the LDS (idle after the last K-step). acc[a][b][e] is y[r][c]
 // with c = lane % 16 + 16 b + wn 16 TN within the tile's first 128 w rows (b < TN) or, for acc[a][TN + b], the same
-// position in its second 128, and tile row r = wm (256 / WM) + a 16 + 4 (lane / 16) + e. A
+// position in its second 128, and tile row r = wm (BM / WM) + a 16 + 4 (lane / 16) + e. A
 // 128-column half of the tile at a time, each wave writes its scaled results as floats into a [256][kEpiStride] LDS
 // tile (the two half-waves' rows, 4 apart, fall on disjoint banks); then each thread takes 8 consecutive columns of
 // a row, so the output, and with kGateAdd the residual, moves in 16-byte accesses, 16 threads to a row's 256 bytes.
 // The results round to bf16 once, at the end, as they would written straight from the registers.
-template <int BM, int WM, int WN, int MODE, int EPI, int TM, int TN, typename Acc>
+template <int BM, int BN, int WM, int WN, int MODE, int EPI, int TM, int TN, typename Acc>
 __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* smem, uint32_t M, uint32_t N,
                                               uint32_t m0, uint32_t w_lo, uint32_t w_hi,
                                               const float* __restrict__ scale, const float* __restrict__ xscale,
@@ -152,8 +154,9 @@ __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* s
     constexpr uint32_t kThreads = WM * WN * 64;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, wm = wave / WN, wn = wave % WN;
     const uint32_t rl = lane % 16u;
-    constexpr uint32_t kEpiStride = kBN + 8u; // floats a staged row: 4 rows apart = 32 banks apart
-    static_assert(BM * kEpiStride * sizeof(float) <= GemmRing<BM, MODE == 0>::kBytes, "the staged half-tile fits in the LDS");
+    constexpr uint32_t kEpiStride = BN + 8u; // floats a staged row: 4 rows apart = 32 banks apart
+    static_assert(BM * kEpiStride * sizeof(float) <= GemmRing<BM, BN, MODE == kW8A16>::kBytes,
+                  "the staged half-tile fits in the LDS");
     constexpr int kHalves = EPI == kSwiGLU ? 1 : 2;
     float* const stage = reinterpret_cast<float*>(smem);
     lds_barrier(); // every wave is done with the last K-step's fragments
@@ -185,8 +188,8 @@ __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* s
         lds_barrier();
         // Output column of staged column 0: the tile's gate columns (SwiGLU), else its first or second 128 columns.
         const uint32_t col0 = hv == 0 ? w_lo : w_hi;
-        for (uint32_t q = tid; q < uint32_t(BM) * 16u; q += kThreads) {
-            const uint32_t r = q >> 4, c8 = (q & 15u) * 8u, row = m0 + r;
+        for (uint32_t q = tid; q < uint32_t(BM) * (BN / 8u); q += kThreads) {
+            const uint32_t r = q / (BN / 8u), c8 = (q % (BN / 8u)) * 8u, row = m0 + r;
             if (row >= M)
                 break; // rows grow with q
             const float4 v0 = *reinterpret_cast<const float4*>(stage + r * kEpiStride + c8);
@@ -221,12 +224,12 @@ __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* s
     }
 }
 
-// WM x WN wavefronts: wave (wm, wn) computes rows wm * (256 / WM) ... of the tile against its TN gate column tiles
+// WM x WN wavefronts: wave (wm, wn) computes rows wm * (BM / WM) ... of the tile against its TN gate column tiles
 // (16 columns each, from wn * 16 TN) and the TN matching up column tiles, on 16 x 16 MFMA tiles
 // (v_mfma_f32_16x16x32_bf16, v_mfma_i32_16x16x64_i8). Every LDS row holds 128 bytes of k: 64 k of bf16 or 128 k of
 // int8, so a K-step is 64 or 128 k.
-template <int BM, int WM, int WN, int MODE, int EPI>
-__global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
+template <int BM, int BN, int WM, int WN, int MODE, int EPI>
+__global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
     const void* __restrict__ xv, const void* __restrict__ wv, const float* __restrict__ scale,
     const float* __restrict__ xscale, uint16_t* __restrict__ out, uint32_t M, uint32_t N, uint32_t K, uint32_t mt,
     uint32_t nt, GemmGate gg)
@@ -237,20 +240,21 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     constexpr uint32_t kKS = 128u / kEA;                  // k of a K-step
     using Acc = typename std::conditional<MODE == kW8A8, int32x4, floatx4>::type;
     constexpr uint32_t kThreads = WM * WN * 64, kWaves = WM * WN;
-    constexpr int TM = int(BM / WM / 16), TN = int(kBN / WN / 16); // MFMA tiles: rows, and gate (= up) columns
+    constexpr int TM = int(BM / WM / 16), TN = int(BN / WN / 16); // MFMA tiles: rows, and gate (= up) columns
     // Row tiles whose A fragments a sub-step holds: half of them (a sub-step is one 32-k half of the K-step over one
     // half of the wave's rows).
     constexpr int FA = TM / 2;
     extern __shared__ u32x4_t smem[];
-    using Ring = GemmRing<BM, I8>;
+    using Ring = GemmRing<BM, BN, I8>;
     constexpr uint32_t kAChunks = Ring::kAChunks, kAStages = Ring::kAStages, kBStages = Ring::kBStages;
+    constexpr uint32_t kBChunks = Ring::kBChunks, RB = Ring::kBRegs;
     constexpr uint32_t kBBase = kAStages * kAChunks;
     uint32_t tm, tn;
     tile_of<BM>(mt, nt, tm, tn);
     const uint32_t m0 = tm * uint32_t(BM);
     // The tile's two 128-row halves of w (and the output columns they give): gate and up rows, or consecutive rows.
-    const uint32_t w_lo = EPI == kSwiGLU ? tn * kBN : tn * 2u * kBN;
-    const uint32_t w_hi = EPI == kSwiGLU ? N + w_lo : w_lo + kBN;
+    const uint32_t w_lo = EPI == kSwiGLU ? tn * uint32_t(BN) : tn * 2u * BN;
+    const uint32_t w_hi = EPI == kSwiGLU ? N + w_lo : w_lo + uint32_t(BN);
     const uint32_t w_rows = EPI == kSwiGLU ? 2u * N : N;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, wm = wave / WN, wn = wave % WN;
     const uint32_t KT = K / kKS;
@@ -281,7 +285,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     // chunks (256 B-rows x 4 k-chunks; rows 0..127 the gate rows n0.., 128..255 the up rows n + n0..) go BI to a
     // thread: chunk q = tid + kThreads i is k-chunk q % 4 of B-row 4 (G / 2) + 2 ((q / 4) % 2) + G % 2, G = q / 8.
     // Each 8 consecutive lanes thus write two rows whose swizzles differ in parity, i.e. 8 distinct chunk columns.
-    constexpr int BI = int(1024 / kThreads);
+    constexpr int BI = int(BN * 8u / kThreads);
     // N * K < 2^30 (int8) or 2^29 (bf16) is checked on the host.
     const __amdgpu_buffer_rsrc_t rw = buffer_rsrc(wv, uint32_t(w_rows * K * kEB));
     uint32_t b_src[BI], b_lo[BI], b_hi[BI];
@@ -289,7 +293,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     for (int i = 0; i < BI && I8; ++i) {
         const uint32_t q = tid + kThreads * uint32_t(i), kc = q & 3u, G = q >> 3;
         const uint32_t brow = 4u * (G >> 1) + 2u * ((q >> 2) & 1u) + (G & 1u);
-        const uint32_t wrow = brow < kBN ? w_lo + brow : w_hi + (brow - kBN);
+        const uint32_t wrow = brow < uint32_t(BN) ? w_lo + brow : w_hi + (brow - uint32_t(BN));
         const uint32_t sx = (brow >> 1) & 7u;
         b_src[i] = wrow * K + kc * 16u;
         b_lo[i] = brow * 128u + ((2u * kc) ^ sx) * 16u;
@@ -301,7 +305,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
             rb[i] = __builtin_amdgcn_raw_buffer_load_b128(rw, b_src[i], int(kt * kBK), 0);
     };
     char* const lds = reinterpret_cast<char*>(smem);
-    u32x4_t rb[BI];
+    u32x4_t rb[RB][BI]; // tile t's B in set t % RB
     // Piece p of tile kt's B write: half p % 2 of register chunk p / 2, widened and stored.
     auto b_piece = [&](uint32_t kt, const u32x4_t (&rb)[BI], int p) {
         char* B = lds + (kBBase + (kt % kBStages) * kBChunks) * 16u;
@@ -320,7 +324,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     for (int i = 0; i < BD && !I8; ++i) {
         const uint32_t row = (wave * BD + uint32_t(i)) * 8u + (lane >> 3);
         const uint32_t c = (lane & 7u) ^ ((row >> 1) & 7u);
-        const uint32_t wrow = row < kBN ? w_lo + row : w_hi + (row - kBN);
+        const uint32_t wrow = row < uint32_t(BN) ? w_lo + row : w_hi + (row - uint32_t(BN));
         bd_off[i] = wrow * K * kEB + c * 16u;
     }
     auto b_dma = [&](uint32_t kt) {
@@ -354,7 +358,7 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
 #pragma unroll
         for (int t = 0; t < TN; ++t) {
             fb[t] = *reinterpret_cast<const bf16x8_t*>(B + t * kRowBytes);
-            fb[TN + t] = *reinterpret_cast<const bf16x8_t*>(B + kBN * 128 + t * kRowBytes);
+            fb[TN + t] = *reinterpret_cast<const bf16x8_t*>(B + BN * 128 + t * kRowBytes);
         }
     };
     // Sub-step ks's fragments; B only at the start of a k-half (the second sub-step of a half keeps it).
@@ -389,8 +393,8 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     };
     // The same MFMAs with B pieces p0 .. p0 + np - 1 of tile kt placed between them, at even spacing, so the
     // widening's VALU work issues while the matrix core is busy.
-    auto mfmas_b = [&](uint32_t ks, const bf16x8_t (&fa)[FA], const bf16x8_t (&fb)[2 * TN], uint32_t kt, int p0,
-                       int np) {
+    auto mfmas_b = [&](uint32_t ks, const bf16x8_t (&fa)[FA], const bf16x8_t (&fb)[2 * TN], uint32_t kt,
+                       const u32x4_t (&rb)[BI], int p0, int np) {
         constexpr int n = FA * 2 * TN;
         const int t0 = int(ks & 1u) * FA;
 #pragma unroll
@@ -412,15 +416,16 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     // K-step earlier, but between the fragment reads and the MFMAs. At 256 rows the MFMAs set the pace (19,305 x 5376 ->
     // 28,672: 4.72 ms early, 4.63 late); with fewer the loads do.
     constexpr bool kEarlyB = !I8 && BM <= 128;
-    static_assert(DA == DB || DA == DB + 1u, "the order that the waits below count on");
-    static_assert(kEarlyB || (DA == 2 && DB == 1));
-    // Prologue: tile 0 in LDS (its B widened), and the later tiles' loads in flight: with int8 weights tile 1's B to
-    // registers and A to LDS; with kEarlyB tiles 1 .. DB's B and 1 .. DA - 1's A, otherwise tile 1's A.
+    static_assert(I8 || DA == DB || DA == DB + 1u, "the order that the waits below count on");
+    static_assert(kEarlyB || (DB == 1 && DA == RB + 1u));
+    // Prologue: tile 0 in LDS (its B widened), and the later tiles' loads in flight, in the order of the loop: with int8
+    // weights tiles 1 .. RB's B to registers and A to LDS; with kEarlyB tiles 1 .. DB's B and 1 .. DA - 1's A, otherwise
+    // tile 1's A.
     // The explicit wait is needed: the compiler may issue the B loads ahead of the LDS-bound A loads, and then the
     // waits it places for the B registers leave tile 0's A outstanding.
     a_issue(0);
     if constexpr (I8)
-        b_issue(0, rb);
+        b_issue(0, rb[0]);
     else
         b_dma(0);
     __builtin_amdgcn_sched_barrier(0);
@@ -440,11 +445,16 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (I8)
-        b_write(0, rb);
-    if (!kEarlyB && KT > 1) {
-        if constexpr (I8)
-            b_issue(1, rb);
-        a_issue(1);
+        b_write(0, rb[0]);
+    if constexpr (!kEarlyB) {
+#pragma unroll
+        for (uint32_t t = 1; t < DA; ++t) {
+            if (t < KT) {
+                if constexpr (I8)
+                    b_issue(t, rb[t % RB]);
+                a_issue(t);
+            }
+        }
     }
     // The epilogue's kernel arguments are read here, before the barrier: a scalar load still in flight at the loop
     // would turn every LDS wait in it into a full wait (scalar loads complete out of order).
@@ -454,19 +464,20 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
     bf16x8_t fa[2][FA], fb[2][2 * TN];
     frags(0, 0, fa[0], fb[0]);
 
-    // One K-step over tile kt (four sub-steps). With int8 weights, tile kt+1's B is widened from registers into LDS in
-    // pieces placed between the MFMAs of the first two sub-steps; then the wave waits for everything it has in flight
-    // (tile kt+1's A, issued a step ago) and tile kt+2's B goes out. Tile kt+DA's A goes out there too. The barrier
-    // publishing tile kt+1 comes after the third sub-step's MFMAs, and the fourth sub-step's operands are already in
-    // registers: the MFMAs keep running while tile kt+1's first fragments load. A B that streams into LDS goes out
-    // after the barrier (kEarlyB) or the step's last MFMAs, DB steps ahead. LDS stages written after step kt-1's barrier (A's (kt+DA) % kAStages, B's
-    // (kt+DB) % kBStages) were last read before it. The last step is a separate instance (kLast) so that the loop body
-    // has no branch around the barrier: at such a join the compiler's LDS wait would also cover tile kt+1's fragment
-    // reads.
+    // One K-step over tile kt (four sub-steps). With int8 weights, tile kt+1's B is widened from registers (set
+    // (kt + 1) % RB) into LDS in pieces placed between the MFMAs of the first two sub-steps; then the wave waits for
+    // tile kt+1's A and tile kt+1+RB's B goes out into the same registers. Tile kt+DA's A goes out there too. The
+    // barrier publishing tile kt+1 comes after the third sub-step's MFMAs, and the fourth sub-step's operands are
+    // already in registers: the MFMAs keep running while tile kt+1's first fragments load. A B that streams into LDS
+    // goes out after the barrier (kEarlyB) or the step's last MFMAs, DB steps ahead. LDS stages written after step
+    // kt-1's barrier (A's (kt+DA) % kAStages, B's (kt+DB) % kBStages) were last read before it. The last step is a
+    // separate instance (kLast) so that the loop body has no branch around the barrier: at such a join the compiler's
+    // LDS wait would also cover tile kt+1's fragment reads.
     // B sets of sub-steps 0..3: one a k-half (0, 0, 1, 1).
     constexpr int B1 = 0, B2 = 1, B3 = 1;
-    auto kstep = [&](uint32_t kt, auto last) {
+    auto kstep = [&](uint32_t kt, auto last, auto set) {
         constexpr bool kLast = decltype(last)::value;
+        u32x4_t(&rbn)[BI] = rb[decltype(set)::value]; // tile kt + 1's B, then tile kt + 1 + RB's
         if constexpr (!I8 && !kEarlyB && !kLast)
             b_dma(kt + 1); // DB is 1
         frags(kt, 1, fa[1], fb[B1]);
@@ -474,18 +485,24 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         if constexpr (kLast || !I8)
             mfmas(0, fa[0], fb[0]);
         else
-            mfmas_b(0, fa[0], fb[0], kt + 1, 0, BI);
+            mfmas_b(0, fa[0], fb[0], kt + 1, rbn, 0, BI);
         frags(kt, 2, fa[0], fb[B2]);
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (kLast || !I8)
             mfmas(1, fa[1], fb[B1]);
         else
-            mfmas_b(1, fa[1], fb[B1], kt + 1, BI, BI);
+            mfmas_b(1, fa[1], fb[B1], kt + 1, rbn, BI, BI);
         if constexpr (!kLast) {
             if constexpr (I8) {
-                __builtin_amdgcn_s_waitcnt(waitcnt_vm(0)); // tile kt+1's A complete too
-                if (kt + 2 < KT)
-                    b_issue(kt + 2, rb);
+                // Tile kt+1's A complete too: the loads after it are those of tiles kt+2 .. kt+DA-1.
+                if (RB > 1 && kt + DA < KT)
+                    __builtin_amdgcn_s_waitcnt(waitcnt_vm(int(RB - 1u) * (BI + AI)));
+                else
+                    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+                __builtin_amdgcn_sched_barrier(0);
+                if (kt + 1u + RB < KT)
+                    b_issue(kt + 1u + RB, rbn);
+                __builtin_amdgcn_sched_barrier(0);
             }
             if (kt + DA < KT)
                 a_issue(kt + DA);
@@ -513,51 +530,73 @@ __global__ __launch_bounds__(kGemmWM * kGemmWN * 64) void gemm_kernel(
         __builtin_amdgcn_sched_barrier(0);
         mfmas(3, fa[1], fb[B3]);
     };
-    for (uint32_t kt = 0; kt + 1 < KT; ++kt)
-        kstep(kt, std::false_type{});
-    kstep(KT - 1, std::true_type{});
+    if constexpr (I8 && RB == 3) {
+        using S0 = std::integral_constant<uint32_t, 0>;
+        using S1 = std::integral_constant<uint32_t, 1>;
+        using S2 = std::integral_constant<uint32_t, 2>;
+        uint32_t kt = 0; // a multiple of 3: the next tile's set is 1
+        for (; kt + 3u < KT; kt += 3u) {
+            kstep(kt, std::false_type{}, S1{});
+            kstep(kt + 1u, std::false_type{}, S2{});
+            kstep(kt + 2u, std::false_type{}, S0{});
+        }
+        if (kt + 1u < KT)
+            kstep(kt, std::false_type{}, S1{});
+        if (kt + 2u < KT)
+            kstep(kt + 1u, std::false_type{}, S2{});
+        kstep(KT - 1u, std::true_type{}, S0{});
+    } else {
+        static_assert(!I8 || RB == 1);
+        using S0 = std::integral_constant<uint32_t, 0>;
+        for (uint32_t kt = 0; kt + 1 < KT; ++kt)
+            kstep(kt, std::false_type{}, S0{});
+        kstep(KT - 1, std::true_type{}, S0{});
+    }
 
-    gemm_epilogue<BM, WM, WN, MODE, EPI, TM, TN>(acc, smem, M, N, m0, w_lo, w_hi, scale, xscale, out, gg);
+    gemm_epilogue<BM, BN, WM, WN, MODE, EPI, TM, TN>(acc, smem, M, N, m0, w_lo, w_hi, scale, xscale, out, gg);
 }
 
 } // namespace mh3
 
 namespace {
 
-// The row tile of a launch of m rows and nt column tiles: the one whose rounds over the CUs (one workgroup each) take
+// The tile of a launch of m rows and nt column tiles of kBN: the one whose rounds over the CUs (one workgroup each) take
 // least, the larger of equals. `time` is a round's cost against 256 rows': it falls more slowly than the rows, since a
 // K-step streams the same B and has the same chain of loads, barrier and fragment reads. Measured a K-step at K 14336,
 // bf16, rounds of the whole chip: 1.55, 1.36, 1.05 and 0.68 us at 256, 192, 128 and 64 rows, and on a nearly empty chip
-// 1.27, 1.08, 0.87 and 0.76. Chosen against 256 rows (us): 945 x 14336 -> 5376 bf16 284 -> 186, int8 weights 313 ->
-// 214; 64 rows of the same 278 -> 177 and 300 -> 195; 945 x 5376 -> 21504 231 -> 217; 1537 x 5376 -> 28672 470 -> 423.
-uint32_t row_tile(uint32_t m, uint32_t nt)
+// 1.27, 1.08, 0.87 and 0.76, and 0.37 for the narrow tile (two of its workgroups share a CU: 0.56 on a full chip).
+// Chosen against 256 rows (us): 945 x 14336 -> 5376 bf16 284 -> 186, int8 weights 313 -> 214; 64 rows of the same 278 -> 82
+// and 300 -> 106 (64 x 128 tiles 177 and 195); 945 x 5376 -> 21504 231 -> 217; 1537 x 5376 -> 28672 470 -> 423.
+struct TileChoice {
+    uint32_t rows, cols, time;
+};
+TileChoice choose_tile(uint32_t m, uint32_t nt)
 {
-    constexpr struct {
-        uint32_t rows, time;
-    } kTiles[] = {{256, 100}, {192, 86}, {128, 68}, {64, 55}};
+    constexpr TileChoice kTiles[] = {{256, 128, 100}, {192, 128, 86}, {128, 128, 68}, {64, 128, 55}, {64, 32, 26}};
     const uint64_t cus = uint64_t(std::max(mh3::host::cu_count(), 1));
     uint64_t best = ~0ull;
-    uint32_t rows = 256;
-    for (const auto& t : kTiles) {
-        const uint64_t tiles = (uint64_t(m) + t.rows - 1u) / t.rows * nt, cost = (tiles + cus - 1u) / cus * t.time;
+    TileChoice choice = kTiles[0];
+    for (const TileChoice& t : kTiles) {
+        const uint64_t tiles = (uint64_t(m) + t.rows - 1u) / t.rows * nt * (mh3::kBN / t.cols);
+        const uint64_t cost = (tiles + cus - 1u) / cus * t.time;
         if (cost < best)
-            best = cost, rows = t.rows;
+            best = cost, choice = t;
     }
-    return rows;
+    return choice;
 }
 
-// The launch with row tiles of BM rows.
-template <int BM, int MODE, int EPI>
+// The launch with tiles of BM rows and BN columns (2 BN where the epilogue pairs none).
+template <int BM, int BN, int WN, int MODE, int EPI>
 int launch_tile(const MH3GemmArgs* a, const void* x, const void* w, const float* scale, const float* xscale,
-                uint16_t* out, const mh3::GemmGate& gg, uint32_t nt, mh3_stream_t stream)
+                uint16_t* out, const mh3::GemmGate& gg, mh3_stream_t stream)
 {
     using namespace mh3;
-    constexpr int WM = kGemmWM, WN = kGemmWN;
-    const auto kernel = &gemm_kernel<BM, WM, WN, MODE, EPI>;
-    constexpr size_t kLds = GemmRing<BM, MODE == kW8A16>::kBytes;
+    constexpr int WM = kGemmWM;
+    const auto kernel = &gemm_kernel<BM, BN, WM, WN, MODE, EPI>;
+    constexpr size_t kLds = GemmRing<BM, BN, MODE == kW8A16>::kBytes;
     if (const hipError_t e = host::allow_dynamic_lds(reinterpret_cast<const void*>(kernel), kLds); e != hipSuccess)
         return host::hip_error(e);
-    const uint32_t mt = (a->m + uint32_t(BM) - 1u) / uint32_t(BM);
+    const uint32_t mt = (a->m + uint32_t(BM) - 1u) / uint32_t(BM), nt = a->n / (EPI == kSwiGLU ? BN : 2 * BN);
     hipLaunchKernelGGL(kernel, dim3(mt * nt), dim3(WM * WN * 64), kLds, static_cast<hipStream_t>(stream), x, w, scale,
                        xscale, out, a->m, a->n, a->k, mt, nt, gg);
     return host::check_launch();
@@ -603,15 +642,18 @@ int launch_gemm(const MH3GemmArgs* a, const void* x, const void* w, const float*
     const uint32_t nt = a->n / kCols;
     if (uint64_t((a->m + kBM - 1) / kBM) * nt >= (uint64_t(1) << 31))
         return MH3_ERR_SHAPE;
-    switch (row_tile(a->m, nt)) {
+    const TileChoice tile = choose_tile(a->m, nt);
+    if (tile.cols == 32)
+        return launch_tile<64, 32, 2, MODE, EPI>(a, x, w, scale, xscale, out, gg, stream);
+    switch (tile.rows) {
     case 64:
-        return launch_tile<64, MODE, EPI>(a, x, w, scale, xscale, out, gg, nt, stream);
+        return launch_tile<64, kBN, kGemmWN, MODE, EPI>(a, x, w, scale, xscale, out, gg, stream);
     case 128:
-        return launch_tile<128, MODE, EPI>(a, x, w, scale, xscale, out, gg, nt, stream);
+        return launch_tile<128, kBN, kGemmWN, MODE, EPI>(a, x, w, scale, xscale, out, gg, stream);
     case 192:
-        return launch_tile<192, MODE, EPI>(a, x, w, scale, xscale, out, gg, nt, stream);
+        return launch_tile<192, kBN, kGemmWN, MODE, EPI>(a, x, w, scale, xscale, out, gg, stream);
     default:
-        return launch_tile<256, MODE, EPI>(a, x, w, scale, xscale, out, gg, nt, stream);
+        return launch_tile<256, kBN, kGemmWN, MODE, EPI>(a, x, w, scale, xscale, out, gg, stream);
     }
 }
 

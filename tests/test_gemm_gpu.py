@@ -230,8 +230,8 @@ def test_gemm_i8_768p_every_row(dev):
 @pytest.mark.parametrize("form", ["w8a16", "bf16", "w8a8"])
 @pytest.mark.parametrize("k", [128, 256, 384, 640])
 def test_gemm_row_tiles(dev, form, k):
-    """Every row tile (64 column tiles on 256 CUs: 1021 rows take 256-row tiles, 763 192, 505 128, 255 and 33 64), its
-    last rows missing, at K-step counts around the LDS rings' depths: every element against float64 products, and the
+    """Every tile (64 column tiles on 256 CUs: 1021 rows take 256-row tiles, 763 192, 505 128, 255 64, 33 the narrow
+    one), its last rows missing, at K-step counts around the LDS rings' depths: every element against float64 products, and the
     rows of a smaller batch bit-identical to the same rows of the larger one (the row tile changes no sum's order)."""
     g = torch.Generator(device=dev).manual_seed(k)
     m_max, n = 1021, 64 * 128

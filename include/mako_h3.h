@@ -294,9 +294,9 @@ int mh3_flash_attn_sparse_128(const MH3AttnArgs* args, const uint16_t* q, const 
 /* The same attention with the query cubes of each head scheduled in `order` (int32 [heads][cubes], a permutation of
  * [0, cubes) per head, as mh3_cube_order writes; entries are clamped to [0, cubes), and a non-permutation leaves
  * some cubes unwritten and computes others twice). No counterpart in the reference: it is flash_attn_sparse_128 with
- * a scheduling input. When the cubes and the heads' dense tiles divide into eighths, each XCD takes a contiguous
- * eighth of a head's cubes in this order (otherwise the cube tiles simply follow it), so cubes whose pass lists
- * centre on the same keys run together and share K/V tiles in that XCD's L2. The outputs equal the plain call's up to the softmax's summation
+ * a scheduling input. Each XCD takes a contiguous part of a head's cubes in this order (1, 2, 4 or 8 XCDs share a
+ * head), so cubes whose pass lists centre on the same keys run together and share K/V tiles in that XCD's L2. The
+ * outputs equal the plain call's up to the softmax's summation
  * order. order may not overlap out (MH3_ERR_PARAM) and must be 4-byte aligned. */
 int mh3_flash_attn_sparse_128_ordered(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k,
                                       const uint16_t* v, const int32_t* idx, const int32_t* cnt, const int32_t* order,

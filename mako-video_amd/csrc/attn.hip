@@ -11,7 +11,8 @@
 //   place: no gather or scatter pass.
 // - A workgroup is one (head, 64-row query tile): two waves of 32 queries. Tiles are numbered dense runs of 64 first,
 //   then one per cube; the dense query tiles of every head come first in the grid (they attend every token, ten
-//   times a cube tile's work), then the cube tiles head by head, so one head's K and V stay hot in the MALL.
+//   times a cube tile's work), then the cube tiles head by head (share_of: a few heads at a time), so their K and V stay
+//   hot in the MALL.
 // - Scores are computed transposed, S^T = K Q^T (keys as the MFMA's M, queries as N): the accumulator puts all of
 //   a query's keys in one lane and its lane + 32 twin, so the softmax's row maximum and sum are in-lane plus one
 //   cross-half exchange, and the rescale of a query's output is one factor per lane.
@@ -20,10 +21,10 @@
 //   16-key chunk c is key 32 (c / 2) + 16 (c % 2) + 8 (p % 8 / 4) + 4 (p / 8) + p % 4.
 // - K and V tiles (64 rows each, 32 KB) go from global memory straight into LDS (buffer_load ... lds), one stage: four
 //   workgroups share a CU, and one's loads arrive while the others compute. (Two stages, and the next tile's K during
-//   P V with its V during the scores, measured slower.) Each lane fetches whichever source chunk its LDS slot holds, so the
-//   layouts are free, with one constraint from the address unit: the four lanes of a quad must fetch one aligned
-//   64-byte piece (a quad spread over four rows is four accesses, and held the K/V stream to about 16 bytes a clock a
-//   CU). K is 256-byte rows whose 16-byte chunks are XOR-swizzled by the row (operand reads of 16 rows hit distinct
+//   P V with its V during the scores, measured slower.) Each lane fetches whichever source chunk its LDS slot holds,
+//   so the layouts are free, with one constraint from the address unit: the four lanes of a quad must fetch one
+//   aligned 64-byte piece (a quad spread over four rows is four accesses, and held the K/V stream to about 16 bytes a
+//   clock a CU). K is 256-byte rows whose 16-byte chunks are XOR-swizzled by the row (operand reads of 16 rows hit distinct
 //   banks); V is 1 KB blocks of 4 keys whose 64-byte pieces are interleaved, read with ds_read_b64_tr_b16. That
 //   instruction hands lane i of a 16-lane group element i & 3 of the 8-byte rows named by lanes (i >> 2) + 4 j,
 //   j = 0..3: with lane L naming key (L >> 2)'s columns d0 + 4 (L & 3) .. + 3, lane i receives column d0 + i of four
@@ -32,16 +33,16 @@
 // - Each cube tile walks its pass list from a rotated start (position rank mod S of S, S the cube workgroups an XCD
 //   holds at once, rank the tile's place in its XCD's sequence), wrapping round. The XCD's resident tiles then sweep
 //   the key cubes together, so a K/V tile one of them fetches is still in L2 when the others that selected it reach
-//   it: the L2 hit rate at 768p went from 11-15% to 29-35% and the L2 misses fell by a fifth, for 2.4% less time
-//   (the DMA latency of each tile also bounds the kernel). The first 4 S tiles of an XCD walk from the start of their
-//   lists instead: they start in step (the whole first round at once, and the next rounds nearly so), and tiles in
-//   step share their K/V tiles by walking together. 5 heads at 768p: 7.37-7.40 ms against 7.96-7.98 rotated from
-//   the first tile and 7.73-7.75 never rotated; 40 heads: 54.0-54.4 against 54.2-54.6 (68.1 never rotated).
+//   it: the L2 hit rate at 768p went from 11-15% to 29-35% and the L2 misses fell by a fifth, for 2.4% less time.
+//   The first 4 S tiles of an XCD walk from the start of their lists instead: they start in step (the whole first round
+//   at once, and the next rounds nearly so), and tiles in step share their K/V tiles by walking together. 5 heads at
+//   768p: 7.37-7.40 ms against 7.96-7.98 rotated from the first tile and 7.73-7.75 never rotated; 40 heads: 54.0-54.4
+//   against 54.2-54.6 (68.1 never rotated).
 // - A grid that is not a multiple of 4 in every direction leaves cubes at its edge with few tokens (16 of 64 slots in a
 //   one-frame image, 32 or less in 37% of the cubes of 37 x 17 x 30). The PACK kernel walks a list's whole cubes first
 //   and then its other cubes' tokens in groups of 16, four groups of any cubes to a key tile, so key tiles are full but
-//   for the last; queries are numbered by token too, so a wave that none falls to only loads. 37 x 17 x 30, 56 heads, ratio
-//   0.1: 3.35 -> 2.22 ms, every cube selected 22.3 -> 16.3 (together with the loads' addresses worked out without
+//   for the last; queries are numbered by token too, so a wave that none falls to only loads. 37 x 17 x 30, 56 heads,
+//   ratio 0.1: 3.35 -> 2.22 ms, every cube selected 22.3 -> 16.3 (together with the loads' addresses worked out without
 //   branches); 1 x 43 x 84, 40 heads, ratio 0.5: 3.64 -> 1.05. Fragment reads ahead and the exponentials between the
 //   P V MFMAs then took these to 2.07, 15.5 and 0.93.
 // - Softmax in base 2 with the scale folded into the exponent. A query's running maximum moves only when a tile
@@ -75,8 +76,8 @@ struct AttnParams {
     uint32_t gt, gh, gw, ch, cw, plane; // plane = ch * cw cubes a frame group
     uint32_t cubes, heads, n_dense, nd; // nd: dense tiles of 64 rows
     uint32_t layout, out_stride;
-    // The workgroup-to-tile map: `share` XCDs take a head's cube tiles in contiguous parts of `per`, `groups` = 8 / share
-    // heads run at once; XCD x takes the dense tiles x dense_per .. of all heads' in turn.
+    // The workgroup-to-tile map: `share` XCDs take a head's cube tiles in contiguous parts of `per`, and `groups` =
+    // 8 / share heads run at once; XCD x takes the dense tiles x dense_per .. of all heads' in turn.
     uint32_t share, groups, per, dense_per;
     uint32_t sweep; // cube workgroups an XCD runs at once (0: pass lists in plain order)
     FastDiv div_plane, div_cw; // c / plane and c / cw by multiply-high: a key tile's cube coordinates cost a few
@@ -142,7 +143,10 @@ __device__ __forceinline__ uint64_t slot_row(const AttnParams& p, const Tile& r,
 // The tokens of a cube tile (none of another), and the row, from the tile's base, of its i-th token counted without the
 // padding (i < 64). A division by 1 .. 4 is a multiplication by 128 / d rounded up and a shift (exact for i < 64).
 __device__ __forceinline__ uint32_t tile_tokens(const Tile& r) { return r.lim_t * r.lim_y * r.lim_x; }
-__device__ __forceinline__ uint32_t small_recip(uint32_t d) { return d == 1u ? 128u : d == 2u ? 64u : d == 3u ? 43u : 32u; }
+__device__ __forceinline__ uint32_t small_recip(uint32_t d)
+{
+    return d == 1u ? 128u : d == 2u ? 64u : d == 3u ? 43u : 32u;
+}
 struct TokenRows {
     uint32_t mx, nx, my, ny, sy, st; // reciprocals and limits of x and y; rows a step in y and t takes
     __device__ __forceinline__ TokenRows(const AttnParams& p, const Tile& r)
@@ -278,7 +282,8 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
         k_chunk[u] = 16u * (k_pos ^ (4u * u + k_row));
     auto rsrc_of = [&](const uint16_t* head, uint64_t row) {
         return __builtin_amdgcn_make_buffer_rsrc(
-            reinterpret_cast<char*>(const_cast<uint16_t*>(head)) + row * p.row_stride * 2ull, 0, int(kRecords), kRsrcFlags);
+            reinterpret_cast<char*>(const_cast<uint16_t*>(head)) + row * p.row_stride * 2ull, 0, int(kRecords),
+            kRsrcFlags);
     };
     // Starts tile t's loads; returns its key mask (bit l: slot l is a token). A cube here is whole (a call whose grid
     // has padding takes the kernel with PACK, which gives it only whole cubes); a dense run may end early.
@@ -516,7 +521,8 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
                 whole[k] = tile_full(tl);
                 n_groups[k] = whole[k] ? 0u : (tile_tokens(tl) + 15u) / 16u; // 0 .. 3
                 const uint32_t nw = uint32_t(__popcll(__ballot(whole[k])));
-                const uint32_t ng = uint32_t(__popcll(__ballot(n_groups[k] & 1u)) + 2 * __popcll(__ballot(n_groups[k] & 2u)));
+                const uint32_t ng = uint32_t(__popcll(__ballot(n_groups[k] & 1u)) +
+                                             2 * __popcll(__ballot(n_groups[k] & 2u)));
                 if (lane == 0 && 2u * k + wave < runs) {
                     counts[2u * (2u * k + wave)] = nw;
                     counts[2u * (2u * k + wave) + 1u] = ng;
@@ -539,7 +545,8 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
                     n_group += ng;
                 }
                 at_w += uint32_t(__popcll(__ballot(whole[k]) & below));
-                at_g += uint32_t(__popcll(__ballot(n_groups[k] & 1u) & below) + 2 * __popcll(__ballot(n_groups[k] & 2u) & below));
+                at_g += uint32_t(__popcll(__ballot(n_groups[k] & 1u) & below) +
+                                 2 * __popcll(__ballot(n_groups[k] & 2u) & below));
                 if (whole[k])
                     seg[at_w] = word[k];
                 for (uint32_t g = 0; g < n_groups[k]; ++g)

@@ -565,8 +565,8 @@ namespace {
 // K-step streams the same B and has the same chain of loads, barrier and fragment reads. Measured a K-step at K 14336,
 // bf16, rounds of the whole chip: 1.55, 1.36, 1.05 and 0.68 us at 256, 192, 128 and 64 rows, and on a nearly empty chip
 // 1.27, 1.08, 0.87 and 0.76, and 0.37 for the narrow tile (two of its workgroups share a CU: 0.56 on a full chip).
-// Chosen against 256 rows (us): 945 x 14336 -> 5376 bf16 284 -> 186, int8 weights 313 -> 214; 64 rows of the same 278 -> 82
-// and 300 -> 106 (64 x 128 tiles 177 and 195); 945 x 5376 -> 21504 231 -> 217; 1537 x 5376 -> 28672 470 -> 423.
+// Chosen against 256 rows (us): 945 x 14336 -> 5376 bf16 284 -> 186, int8 weights 313 -> 214; 64 rows of the same
+// 278 -> 82 and 300 -> 106 (64 x 128 tiles 177 and 195); 945 x 5376 -> 21504 231 -> 217; 1537 x 5376 -> 28672 470 -> 423.
 struct TileChoice {
     uint32_t rows, cols, time;
 };

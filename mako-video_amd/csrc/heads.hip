@@ -16,7 +16,7 @@
 //   (the norm factor is the group's).
 // - The workgroup stages the two norm weight vectors and its rows' cos / sin tables in LDS once.
 // - A padding slot of the cube map writes zeros and reads nothing.
-// mh3_heads_partial_pool adds cube_pool to the same pass (heads_pool_kernel, workgroups of one cube each): the selector's
+// mh3_heads_partial_pool adds cube_pool to the same pass (heads_pool_kernel, a cube a workgroup): the selector's
 // cube means come from the values as they are stored, so q and k are not read back from HBM.
 #include "mh3_common.hpp"
 
@@ -126,8 +126,8 @@ __device__ __forceinline__ void stage_weights(float* wt, const float* qw, const 
 
 // Output rows r0 .. r0 + nr - 1 (nr <= rows_per_block) by a workgroup of kHeadsThreads. LDS: the norm weights w [2][128]
 // (q, then k); the rows' model rows src [rows_per_block] (-1: padding); their cos and sin tables [rows_per_block][half]
-// each.
-__device__ __forceinline__ void heads_rows(const HeadsParams& p, uint32_t r0, uint32_t nr, float* lds)
+// each. The parameters go by value: through a reference the compiler reloads them (768p: 1.64 against 1.51 ms).
+__device__ __forceinline__ void heads_rows(const HeadsParams p, uint32_t r0, uint32_t nr, float* lds)
 {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, part = lane & 15u, group = tid >> 4;
     float* wt = lds;
@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kHeadsThreads) void heads_kernel(HeadsParams p)
 // A wave takes four consecutive head vectors (one a 16-lane group, so a load reads 1 KB of a row) and one dx, so two
 // sets of four waves cover the workgroup's 8 vectors and the four dx sums meet in LDS. HBM-bound where the cubes fill
 // the chip; a workgroup that took a whole cube left it idle on short clips (30 cubes, 40 heads: 177 us, now 30) and
-// unevenly filled at 960 x 544 (400 cubes, 56 heads: 461 -> 417 us; 2016 cubes, 40 heads: 1.63 -> 1.53 ms). The
+// unevenly filled at 960 x 544 (400 cubes, 56 heads: 461 -> 401 us; 2016 cubes, 40 heads: 1.63 -> 1.53 ms). The
 // tables' loads are all issued before the first is stored (one after the other, each behind its map entry, they cost
 // 8% at 2016 cubes). Two to six workgroups a cube, each looping over its vectors, measured between the two.
 // The rows before and after the cubes' (the dense rows) go to workgroups of the same launch.
@@ -486,11 +486,14 @@ extern "C" int mh3_heads_partial_pool(const MH3HeadsArgs* args, const MH3CubeArg
     pp.video0 = uint32_t(cb.row0), pp.video1 = uint32_t(cb.row0 + span);
     pp.cube_wgs = uint32_t(ncubes) * pp.parts;
     pp.wgs0 = (pp.video0 + p.rows_per_block - 1u) / p.rows_per_block;
-    const uint64_t wgs = uint64_t(pp.cube_wgs) + pp.wgs0 + (p.rows - pp.video1 + p.rows_per_block - 1u) / p.rows_per_block;
-    const size_t lds = (256u + 64u + 2u * std::max(64u * p.half, 8u) + 8u * kPoolThreads) * sizeof(float); // 26 KB at rot 96
+    const uint64_t wgs =
+        uint64_t(pp.cube_wgs) + pp.wgs0 + (p.rows - pp.video1 + p.rows_per_block - 1u) / p.rows_per_block;
+    // The weights, source rows and tables, and two float4 of partial sums a thread: 42 KB at rot 96.
+    const size_t lds = (256u + 64u + 2u * std::max(64u * p.half, 8u) + 8u * kPoolThreads) * sizeof(float);
     if (const hipError_t e = host::allow_dynamic_lds(reinterpret_cast<const void*>(&heads_pool_kernel), lds);
         e != hipSuccess)
         return host::hip_error(e);
-    hipLaunchKernelGGL(heads_pool_kernel, dim3(uint32_t(wgs)), dim3(kPoolThreads), lds, static_cast<hipStream_t>(stream), pp);
+    hipLaunchKernelGGL(heads_pool_kernel, dim3(uint32_t(wgs)), dim3(kPoolThreads), lds,
+                       static_cast<hipStream_t>(stream), pp);
     return host::check_launch();
 }

@@ -417,7 +417,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
     // 28,672: 4.72 ms early, 4.63 late); with fewer the loads do.
     constexpr bool kEarlyB = !I8 && BM <= 128;
     static_assert(I8 || DA == DB || DA == DB + 1u, "the order that the waits below count on");
-    static_assert(kEarlyB || (DB == 1 && DA == RB + 1u));
+    static_assert(kEarlyB || DB == 1);
+    static_assert(!I8 || DA == RB + 1u);
     // Prologue: tile 0 in LDS (its B widened), and the later tiles' loads in flight, in the order of the loop: with int8
     // weights tiles 1 .. RB's B to registers and A to LDS; with kEarlyB tiles 1 .. DB's B and 1 .. DA - 1's A, otherwise
     // tile 1's A.
@@ -500,12 +501,17 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
                 else
                     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
                 __builtin_amdgcn_sched_barrier(0);
-                if (kt + 1u + RB < KT)
-                    b_issue(kt + 1u + RB, rbn);
-                __builtin_amdgcn_sched_barrier(0);
             }
-            if (kt + DA < KT)
+            // One branch for both (DA is RB + 1): under two the compiler must allow for B's loads without A's behind
+            // them, and its wait for B's registers in the next step drains A's as well (fc2 19,305 x 14336 -> 5376:
+            // 2497 us so, 2460 under one; 945 rows 223 and 211).
+            if (kt + DA < KT) {
+                if constexpr (I8) {
+                    b_issue(kt + DA, rbn);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
                 a_issue(kt + DA);
+            }
             __builtin_amdgcn_sched_barrier(0); // the waits count these loads: none moves past here
         }
         frags(kt, 3, fa[1], fb[B3]);

@@ -437,8 +437,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
                 b_dma(t);
             if (t < DA && t < KT)
                 a_issue(t);
+            __builtin_amdgcn_sched_barrier(0); // the loop's waits count on this order
         }
-        __builtin_amdgcn_sched_barrier(0);
     }
     if (kEarlyB && KT > DA) // the loads after tile 0's
         __builtin_amdgcn_s_waitcnt(waitcnt_vm(int(DB) * BD + int(DA - 1u) * AI));
@@ -447,23 +447,28 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (I8)
         b_write(0, rb[0]);
-    if constexpr (!kEarlyB) {
+    bf16x8_t fa[2][FA], fb[2][2 * TN]; // fragment double buffers: A by sub-step parity, B by k-half (shared by its two)
+    // Tiles 1 .. DA - 1's loads (all of them there: every tile exists), tile 0's barrier and first fragments.
+    auto begin = [&](auto all) {
+        if constexpr (!kEarlyB) {
 #pragma unroll
-        for (uint32_t t = 1; t < DA; ++t) {
-            if (t < KT) {
-                if constexpr (I8)
-                    b_issue(t, rb[t % RB]);
-                a_issue(t);
+            for (uint32_t t = 1; t < DA; ++t) {
+                if (decltype(all)::value || t < KT) {
+                    if constexpr (I8) {
+                        b_issue(t, rb[t % RB]);
+                        __builtin_amdgcn_sched_barrier(0);
+                    }
+                    a_issue(t);
+                    __builtin_amdgcn_sched_barrier(0); // the loop's waits count on this order
+                }
             }
         }
-    }
-    // The epilogue's kernel arguments are read here, before the barrier: a scalar load still in flight at the loop
-    // would turn every LDS wait in it into a full wait (scalar loads complete out of order).
-    asm volatile("" ::"s"(scale), "s"(xscale), "s"(out), "s"(gg.gate), "s"(gg.set_of_row));
-    lds_barrier();
-    // Fragment double buffers: A by sub-step parity, B by k-half (a half's two sub-steps share one B set).
-    bf16x8_t fa[2][FA], fb[2][2 * TN];
-    frags(0, 0, fa[0], fb[0]);
+        // The epilogue's kernel arguments are read here, before the barrier: a scalar load still in flight at the loop
+        // would turn every LDS wait in it into a full wait (scalar loads complete out of order).
+        asm volatile("" ::"s"(scale), "s"(xscale), "s"(out), "s"(gg.gate), "s"(gg.set_of_row));
+        lds_barrier();
+        frags(0, 0, fa[0], fb[0]);
+    };
 
     // One K-step over tile kt (four sub-steps). With int8 weights, tile kt+1's B is widened from registers (set
     // (kt + 1) % RB) into LDS in pieces placed between the MFMAs of the first two sub-steps; then the wave waits for
@@ -476,8 +481,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
     // LDS wait would also cover tile kt+1's fragment reads.
     // B sets of sub-steps 0..3: one a k-half (0, 0, 1, 1).
     constexpr int B1 = 0, B2 = 1, B3 = 1;
-    auto kstep = [&](uint32_t kt, auto last, auto set) {
-        constexpr bool kLast = decltype(last)::value;
+    auto kstep = [&](uint32_t kt, auto last, auto set, auto more) {
+        constexpr bool kLast = decltype(last)::value, kMore = decltype(more)::value; // kMore: tile kt + DA exists
         u32x4_t(&rbn)[BI] = rb[decltype(set)::value]; // tile kt + 1's B, then tile kt + 1 + RB's
         if constexpr (!I8 && !kEarlyB && !kLast)
             b_dma(kt + 1); // DB is 1
@@ -496,7 +501,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
         if constexpr (!kLast) {
             if constexpr (I8) {
                 // Tile kt+1's A complete too: the loads after it are those of tiles kt+2 .. kt+DA-1.
-                if (RB > 1 && kt + DA < KT)
+                if (RB > 1 && (kMore || kt + DA < KT))
                     __builtin_amdgcn_s_waitcnt(waitcnt_vm(int(RB - 1u) * (BI + AI)));
                 else
                     __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
@@ -505,7 +510,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
             // One branch for both (DA is RB + 1): under two the compiler must allow for B's loads without A's behind
             // them, and its wait for B's registers in the next step drains A's as well (fc2 19,305 x 14336 -> 5376:
             // 2497 us so, 2460 under one; 945 rows 223 and 211).
-            if (kt + DA < KT) {
+            if (kMore || kt + DA < KT) {
                 if constexpr (I8) {
                     b_issue(kt + DA, rbn);
                     __builtin_amdgcn_sched_barrier(0);
@@ -540,23 +545,40 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
         using S0 = std::integral_constant<uint32_t, 0>;
         using S1 = std::integral_constant<uint32_t, 1>;
         using S2 = std::integral_constant<uint32_t, 2>;
+        using Any = std::false_type;
         uint32_t kt = 0; // a multiple of 3: the next tile's set is 1
+        // The steps whose loads are all there go in a loop without branches around them, entered with all of tiles
+        // 1 .. DA - 1's in flight: with either conditional, the compiler's wait for B's registers at the loop's head
+        // allows for the path with the fewest loads behind them and drains the later tiles' too, which leaves the sets
+        // no use (64 x 14336 -> 5376: 99 us so, 70 without; 64 x 5376 -> 28672 54 and 51).
+        if (KT >= DA + 3u) {
+            begin(std::true_type{});
+            do {
+                kstep(kt, std::false_type{}, S1{}, std::true_type{});
+                kstep(kt + 1u, std::false_type{}, S2{}, std::true_type{});
+                kstep(kt + 2u, std::false_type{}, S0{}, std::true_type{});
+                kt += 3u;
+            } while (kt + 2u + DA < KT);
+        } else {
+            begin(std::false_type{});
+        }
         for (; kt + 3u < KT; kt += 3u) {
-            kstep(kt, std::false_type{}, S1{});
-            kstep(kt + 1u, std::false_type{}, S2{});
-            kstep(kt + 2u, std::false_type{}, S0{});
+            kstep(kt, std::false_type{}, S1{}, Any{});
+            kstep(kt + 1u, std::false_type{}, S2{}, Any{});
+            kstep(kt + 2u, std::false_type{}, S0{}, Any{});
         }
         if (kt + 1u < KT)
-            kstep(kt, std::false_type{}, S1{});
+            kstep(kt, std::false_type{}, S1{}, Any{});
         if (kt + 2u < KT)
-            kstep(kt + 1u, std::false_type{}, S2{});
-        kstep(KT - 1u, std::true_type{}, S0{});
+            kstep(kt + 1u, std::false_type{}, S2{}, Any{});
+        kstep(KT - 1u, std::true_type{}, S0{}, Any{});
     } else {
         static_assert(!I8 || RB == 1);
         using S0 = std::integral_constant<uint32_t, 0>;
+        begin(std::false_type{});
         for (uint32_t kt = 0; kt + 1 < KT; ++kt)
-            kstep(kt, std::false_type{}, S0{});
-        kstep(KT - 1, std::true_type{}, S0{});
+            kstep(kt, std::false_type{}, S0{}, std::false_type{});
+        kstep(KT - 1, std::true_type{}, S0{}, std::false_type{});
     }
 
     gemm_epilogue<BM, BN, WM, WN, MODE, EPI, TM, TN>(acc, smem, M, N, m0, w_lo, w_hi, scale, xscale, out, gg);
@@ -570,9 +592,10 @@ namespace {
 // least, the larger of equals. `time` is a round's cost against 256 rows': it falls more slowly than the rows, since a
 // K-step streams the same B and has the same chain of loads, barrier and fragment reads. Measured a K-step at K 14336,
 // bf16, rounds of the whole chip: 1.55, 1.36, 1.05 and 0.68 us at 256, 192, 128 and 64 rows, and on a nearly empty chip
-// 1.27, 1.08, 0.87 and 0.76, and 0.37 for the narrow tile (two of its workgroups share a CU: 0.56 on a full chip).
-// Chosen against 256 rows (us): 945 x 14336 -> 5376 bf16 284 -> 186, int8 weights 313 -> 214; 64 rows of the same
-// 278 -> 82 and 300 -> 106 (64 x 128 tiles 177 and 195); 945 x 5376 -> 21504 231 -> 217; 1537 x 5376 -> 28672 470 -> 423.
+// 1.27, 1.08, 0.87 and 0.76, and 0.37 for the narrow tile (two of its workgroups share a CU: 0.56 on a full chip; int8
+// weights 0.31).
+// Chosen against 256 rows (us): 945 x 14336 -> 5376 bf16 284 -> 186, int8 weights 313 -> 211; 64 rows of the same
+// 278 -> 84 and 300 -> 70 (64 x 128 tiles 177 and 195); 945 x 5376 -> 21504 231 -> 217; 1537 x 5376 -> 28672 470 -> 423.
 struct TileChoice {
     uint32_t rows, cols, time;
 };

@@ -265,3 +265,18 @@ def test_gemm_row_tiles(dev, form, k):
     for m in (763, 505, 255, 33):
         for name, a, b in zip(("fc1", "store", "gate_add", "gate_add_f32"), run(m), full):
             assert torch.equal(a, b[:m]), f"{form} {name} k {k} m {m}"
+
+
+@pytest.mark.parametrize("form", ["w8a16", "bf16"])
+@pytest.mark.parametrize("steps", [1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 13])
+def test_gemm_narrow_k_steps(dev, form, steps):
+    """The narrow tile (33 rows of 64 column tiles on 256 CUs) at every K-step count around its rings' depth and its
+    loop's three steps: every element against float64 products, and bit-identical to a larger tile's."""
+    k, n = 64 * steps, 64 * 128
+    g = torch.Generator(device=dev).manual_seed(steps)
+    x = torch.randn((1021, k), generator=g, device=dev).to(torch.bfloat16)
+    wf = (0.02 * torch.randn((2 * n, k), generator=g, device=dev)).to(torch.bfloat16)
+    w, ws = (wf, None) if form == "bf16" else mh.quant_rows_i8(wf)
+    y = mh.gemm(x[:33], w, w_scale=ws, out=nan_filled((33, 2 * n), dev))
+    check_gemm_full(y, x[:33], w, f"{form} k {k}", w_scale=ws)
+    assert torch.equal(y, mh.gemm(x, w, w_scale=ws, out=nan_filled((1021, 2 * n), dev))[:33])

@@ -72,3 +72,12 @@ def test_w8a16_widening_leaves_later_loads_in_flight(code_objects, rows, epi):
     waits = load_waits(loops[0])
     assert waits[-1] == 0 and len(waits) > 1
     assert min(waits[:-1]) >= rows // 64, waits
+
+
+@pytest.mark.parametrize("epi", [0, 1, 2, 3])
+def test_w8a16_narrow_tile_keeps_two_later_tiles_in_flight(code_objects, epi):
+    # Three register sets of w: a step's loads are one of w and two of x, and no wait of the three steps that the loop
+    # without branches holds may leave fewer than the two later tiles' six in flight.
+    loops = k_loops(instructions(code_objects, f"gemm_kernelILi64ELi32ELi2ELi2ELi0ELi{epi}E"))
+    waits = max((load_waits(body) for body in loops), key=min)
+    assert len(waits) >= 3 and min(waits) >= 6, [load_waits(body) for body in loops]

@@ -50,6 +50,7 @@
 #include "mh3_common.hpp"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace mh3 {
 namespace {
@@ -80,6 +81,7 @@ struct AttnParams {
     // 8 / share heads run at once; XCD x takes the dense tiles x dense_per .. of all heads' in turn.
     uint32_t share, groups, per, dense_per;
     uint32_t sweep; // cube workgroups an XCD runs at once (0: pass lists in plain order)
+    uint32_t slots; // workgroups the chip runs at once
     FastDiv div_plane, div_cw; // c / plane and c / cw by multiply-high: a key tile's cube coordinates cost a few
                                // scalar instructions instead of integer divisions
     float scale_log2;    // score scale times log2(e): softmax in base 2
@@ -196,8 +198,9 @@ __device__ __forceinline__ bool tile_full(const Tile& r)
     return r.kind == 0 ? r.lim_t == 64u : (r.kind != 3 && r.lim_t == 4u && r.lim_y == 4u && r.lim_x == 4u);
 }
 
-// kAhead: how many fragments are read ahead of their MFMAs (stream_bound says which of the two a call takes).
-template <bool PACK, int kAhead>
+// PACED: a call bound by the K/V stream past L2 (stream_bound), whose cube tiles read a fragment right before its MFMA;
+// the others read eight ahead.
+template <bool PACK, bool PACED>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams p)
 {
     extern __shared__ __attribute__((aligned(16))) char lds[]; // K, V; with PACK the segment's entries (kSegWords)
@@ -375,8 +378,10 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
     const uint32_t L = lane & 15u, grp = lane >> 4;
     const uint32_t v_lane = 1024u * (grp >> 1) + 32u * (grp & 1u) + 64u * (L >> 2) + 8u * (L & 3u);
 
-    // One tile: its scores, their softmax, and its part of the output.
-    auto attend = [&](uint64_t mask) {
+    // One tile: its scores, their softmax, and its part of the output; ahead: how many fragments are read ahead of their
+    // MFMAs.
+    auto attend = [&](uint64_t mask, auto ahead) {
+        constexpr int kAhead = decltype(ahead)::value;
         const char* ks = lds;
         const char* vs = lds + 16384u + v_lane;
         auto read_k = [&](int j) { // key block j % 2, d chunk j / 2
@@ -482,7 +487,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
     };
     // `count` tiles: entry(v) names tile v, fetched while the tile before it is in flight; load(v, entry) starts its
     // loads and returns its key mask.
-    auto walk = [&](uint32_t count, auto entry, auto load) {
+    auto walk = [&](uint32_t count, auto entry, auto load, auto ahead) {
         uint32_t next = count ? entry(0u) : 0u;
         for (uint32_t v = 0; v < count; ++v) {
             const uint64_t mask = load(v, next);
@@ -491,87 +496,113 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
             wait_vm0();
             lds_barrier(); // tile v is in LDS for every wave
             if (!PACK || !idle)
-                attend(mask);
+                attend(mask, ahead);
             lds_barrier(); // every wave is done with it before it is overwritten
         }
     };
-    if constexpr (!PACK) {
-        walk(
-            n_sel + p.nd,
-            [&](uint32_t e) {
-                const uint32_t c = e < n_sel ? key_cube(e) : 0u;
-                return e >= n_sel ? e - n_sel : c == kNoTile ? kNoTile : p.nd + c;
-            },
-            [&](uint32_t, uint32_t tile) { return dma_tile(tile); });
-    } else {
-        // The entries a segment at a time: its whole cubes from the front of seg[], and the groups of 16 tokens of the
-        // others from the back, each in list order.
-        uint32_t* const seg = reinterpret_cast<uint32_t*>(lds + kStageBytes);
-        uint32_t* const counts = seg + kSegWords; // per 64 entries: whole cubes, groups
-        for (uint32_t s0 = 0;; s0 += kSegEntries) {
-            const uint32_t n_seg = min(kSegEntries, n_sel - min(s0, n_sel)), runs = (n_seg + 63u) / 64u;
-            const bool last = s0 + kSegEntries >= n_sel;
-            uint32_t word[kSegEntries / kAttnThreads], n_groups[kSegEntries / kAttnThreads];
-            bool whole[kSegEntries / kAttnThreads];
-#pragma unroll
-            for (uint32_t k = 0; k < kSegEntries / kAttnThreads; ++k) {
-                const uint32_t e = kAttnThreads * k + tid;
-                word[k] = e < n_seg ? key_cube(s0 + e) : kNoTile;
-                const Tile tl = make_tile(p, word[k] == kNoTile ? kNoTile : p.nd + word[k]);
-                whole[k] = tile_full(tl);
-                n_groups[k] = whole[k] ? 0u : (tile_tokens(tl) + 15u) / 16u; // 0 .. 3
-                const uint32_t nw = uint32_t(__popcll(__ballot(whole[k])));
-                const uint32_t ng = uint32_t(__popcll(__ballot(n_groups[k] & 1u)) +
-                                             2 * __popcll(__ballot(n_groups[k] & 2u)));
-                if (lane == 0 && 2u * k + wave < runs) {
-                    counts[2u * (2u * k + wave)] = nw;
-                    counts[2u * (2u * k + wave) + 1u] = ng;
-                }
-            }
-            lds_barrier();
-            uint32_t n_whole = 0, n_group = 0;
-#pragma unroll
-            for (uint32_t k = 0; k < kSegEntries / kAttnThreads; ++k) {
-                const uint64_t below = lanes_below(int(lane));
-                uint32_t at_w = n_whole, at_g = n_group;
-#pragma unroll
-                for (uint32_t w = 0; w < 2; ++w) {
-                    if (2u * k + w >= runs)
-                        continue;
-                    const uint32_t nw = counts[2u * (2u * k + w)], ng = counts[2u * (2u * k + w) + 1u];
-                    at_w += w < wave ? nw : 0u;
-                    at_g += w < wave ? ng : 0u;
-                    n_whole += nw;
-                    n_group += ng;
-                }
-                at_w += uint32_t(__popcll(__ballot(whole[k]) & below));
-                at_g += uint32_t(__popcll(__ballot(n_groups[k] & 1u) & below) +
-                                 2 * __popcll(__ballot(n_groups[k] & 2u) & below));
-                if (whole[k])
-                    seg[at_w] = word[k];
-                for (uint32_t g = 0; g < n_groups[k]; ++g)
-                    seg[kSegWords - 1u - (at_g + g)] = word[k] | g << 30;
-            }
-            lds_barrier();
-            n_whole = __builtin_amdgcn_readfirstlane(n_whole);
-            n_group = __builtin_amdgcn_readfirstlane(n_group);
-            const uint32_t packed = (n_group + 3u) / 4u;
+    auto run = [&](auto ahead) {
+        if constexpr (!PACK) {
             walk(
-                n_whole + packed + (last ? p.nd : 0u),
-                [&](uint32_t v) -> uint32_t {
-                    const uint32_t g0 = 4u * (v - n_whole); // of a packed tile: its first group
-                    return seg[v < n_whole              ? v
-                               : v - n_whole < packed ? kSegWords - 1u - min(g0 + (lane & 3u), n_group - 1u)
-                                                      : 0u];
+                n_sel + p.nd,
+                [&](uint32_t e) {
+                    const uint32_t c = e < n_sel ? key_cube(e) : 0u;
+                    return e >= n_sel ? e - n_sel : c == kNoTile ? kNoTile : p.nd + c;
                 },
-                [&](uint32_t v, uint32_t word) {
-                    if (v - n_whole < packed)
-                        return dma_packed(word, min(n_group - 4u * (v - n_whole), 4u));
-                    return dma_tile(v < n_whole ? p.nd + __builtin_amdgcn_readfirstlane(word) : v - n_whole - packed);
-                });
-            if (last)
-                break;
+                [&](uint32_t, uint32_t tile) { return dma_tile(tile); }, ahead);
+        } else {
+            // The entries a segment at a time: its whole cubes from the front of seg[], and the groups of 16 tokens of the
+            // others from the back, each in list order.
+            uint32_t* const seg = reinterpret_cast<uint32_t*>(lds + kStageBytes);
+            uint32_t* const counts = seg + kSegWords; // per 64 entries: whole cubes, groups
+            for (uint32_t s0 = 0;; s0 += kSegEntries) {
+                const uint32_t n_seg = min(kSegEntries, n_sel - min(s0, n_sel)), runs = (n_seg + 63u) / 64u;
+                const bool last = s0 + kSegEntries >= n_sel;
+                uint32_t word[kSegEntries / kAttnThreads], n_groups[kSegEntries / kAttnThreads];
+                bool whole[kSegEntries / kAttnThreads];
+    #pragma unroll
+                for (uint32_t k = 0; k < kSegEntries / kAttnThreads; ++k) {
+                    const uint32_t e = kAttnThreads * k + tid;
+                    word[k] = e < n_seg ? key_cube(s0 + e) : kNoTile;
+                    const Tile tl = make_tile(p, word[k] == kNoTile ? kNoTile : p.nd + word[k]);
+                    whole[k] = tile_full(tl);
+                    n_groups[k] = whole[k] ? 0u : (tile_tokens(tl) + 15u) / 16u; // 0 .. 3
+                    const uint32_t nw = uint32_t(__popcll(__ballot(whole[k])));
+                    const uint32_t ng = uint32_t(__popcll(__ballot(n_groups[k] & 1u)) +
+                                                 2 * __popcll(__ballot(n_groups[k] & 2u)));
+                    if (lane == 0 && 2u * k + wave < runs) {
+                        counts[2u * (2u * k + wave)] = nw;
+                        counts[2u * (2u * k + wave) + 1u] = ng;
+                    }
+                }
+                lds_barrier();
+                uint32_t n_whole = 0, n_group = 0;
+    #pragma unroll
+                for (uint32_t k = 0; k < kSegEntries / kAttnThreads; ++k) {
+                    const uint64_t below = lanes_below(int(lane));
+                    uint32_t at_w = n_whole, at_g = n_group;
+    #pragma unroll
+                    for (uint32_t w = 0; w < 2; ++w) {
+                        if (2u * k + w >= runs)
+                            continue;
+                        const uint32_t nw = counts[2u * (2u * k + w)], ng = counts[2u * (2u * k + w) + 1u];
+                        at_w += w < wave ? nw : 0u;
+                        at_g += w < wave ? ng : 0u;
+                        n_whole += nw;
+                        n_group += ng;
+                    }
+                    at_w += uint32_t(__popcll(__ballot(whole[k]) & below));
+                    at_g += uint32_t(__popcll(__ballot(n_groups[k] & 1u) & below) +
+                                     2 * __popcll(__ballot(n_groups[k] & 2u) & below));
+                    if (whole[k])
+                        seg[at_w] = word[k];
+                    for (uint32_t g = 0; g < n_groups[k]; ++g)
+                        seg[kSegWords - 1u - (at_g + g)] = word[k] | g << 30;
+                }
+                lds_barrier();
+                n_whole = __builtin_amdgcn_readfirstlane(n_whole);
+                n_group = __builtin_amdgcn_readfirstlane(n_group);
+                const uint32_t packed = (n_group + 3u) / 4u;
+                walk(
+                    n_whole + packed + (last ? p.nd : 0u),
+                    [&](uint32_t v) -> uint32_t {
+                        const uint32_t g0 = 4u * (v - n_whole); // of a packed tile: its first group
+                        return seg[v < n_whole              ? v
+                                   : v - n_whole < packed ? kSegWords - 1u - min(g0 + (lane & 3u), n_group - 1u)
+                                                          : 0u];
+                    },
+                    [&](uint32_t v, uint32_t word) {
+                        if (v - n_whole < packed)
+                            return dma_packed(word, min(n_group - 4u * (v - n_whole), 4u));
+                        return dma_tile(v < n_whole ? p.nd + __builtin_amdgcn_readfirstlane(word) : v - n_whole - packed);
+                    },
+                    ahead);
+                if (last)
+                    break;
+            }
         }
+    };
+    using Ahead1 = std::integral_constant<int, 1>;
+    using Ahead8 = std::integral_constant<int, 8>;
+    if constexpr (!PACED) {
+        run(Ahead8{});
+    } else {
+        // A dense tile walks every key tile, and in a call of few heads that chain can take as long as all of the cube
+        // tiles: it then reads eight ahead too. That is where it is longer than a workgroup's share of all the call's
+        // walks (the lists' mean from 64 of the head's counts), by an eighth: at that share and below, both paces are
+        // within 2% (5 heads of 2016 cubes, 512 dense rows: ratio 0.02 4.80 -> 4.22 ms, 0.05 5.35 -> 4.75, 0.1
+        // 7.36 and 7.48; 1440 cubes at 0.1 3.87 -> 3.69, 1760 5.43 and 5.44).
+        bool eager = false;
+        if (dense_q) {
+            const int32_t n = p.cnt[uint64_t(h) * p.cubes + (uint64_t(lane) * p.cubes >> 6)];
+            const float mean = wave_sum(float(min(max(n, 0), int32_t(p.out_stride)))) * (1.0f / 64.0f);
+            const float chain = float(p.cubes) + float(p.nd), dense = float(p.nd);
+            const float walks = float(p.heads) * (float(p.cubes) * (mean + dense) + dense * chain);
+            eager = __builtin_amdgcn_readfirstlane(chain * float(p.slots) > 1.125f * walks);
+        }
+        if (eager)
+            run(Ahead8{});
+        else
+            run(Ahead1{});
     }
 
     // Normalize and write the query rows (a gathered cube's padding slots get zeros; other non-tokens nothing).
@@ -696,9 +727,9 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     p.scale_log2 = scale * 1.4426950408889634f;
     const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
     const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0;
-    const auto kernel = pack                                            ? &attn_sparse_kernel<true, 8>
-                        : stream_bound((video + args->n_dense) * 512ull, p) ? &attn_sparse_kernel<false, 1>
-                                                                        : &attn_sparse_kernel<false, 8>;
+    const auto kernel = pack                                                ? &attn_sparse_kernel<true, false>
+                        : stream_bound((video + args->n_dense) * 512ull, p) ? &attn_sparse_kernel<false, true>
+                                                                            : &attn_sparse_kernel<false, false>;
     const void* kern = reinterpret_cast<const void*>(kernel);
     const size_t lds = kStageBytes + (pack ? kSegBytes : 0u);
     if (const hipError_t e = host::allow_dynamic_lds(kern, lds); e != hipSuccess)
@@ -709,7 +740,8 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
             e != hipSuccess)
             return host::hip_error(e);
         // The sweep period: the cube workgroups an XCD holds at once (half or twice that measured slower).
-        p.sweep = uint32_t(uint64_t(std::max(per_cu, 1)) * uint32_t(host::cu_count()) / 8u);
+        p.slots = uint32_t(std::max(per_cu, 1)) * uint32_t(host::cu_count());
+        p.sweep = p.slots / 8u;
     }
     hipLaunchKernelGGL(kernel, dim3(uint32_t(blocks)), dim3(kAttnThreads), lds, static_cast<hipStream_t>(stream), p);
     return host::check_launch();

@@ -388,3 +388,58 @@ def test_flash_attn_sparse_packed_edges(dev, grid, layout, n_dense, kk):
         tc = torch.zeros((heads, C), dtype=torch.int32, device=dev)
         out = mh.flash_attn_sparse_128(a, q, k, v, ti, tc, out=nan_filled((heads, rows, 128), dev))
         assert bool((out[:, ref[0][0]] == 0).all()), "empty lists"
+
+
+def best_ms(call, runs=12):
+    """The shortest of `runs` timed calls, after two untimed ones."""
+    best = float("inf")
+    for i in range(runs + 2):
+        a, b = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+        a.record()
+        call()
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b)) if i >= 2 else best
+    return best
+
+
+@pytest.mark.parametrize("heads,grid,layout,n_dense,lists", [
+    (2, (32, 52, 52), orc.CUBES_GRID, 70, 27),        # 44 MB of K and V a head: the dense tiles' chains are the call
+    (2, (32, 52, 52), orc.CUBES_GATHERED, 70, 500),   # and here the cube tiles are
+])
+def test_flash_attn_sparse_large_heads(dev, heads, grid, layout, n_dense, lists):
+    """Heads of many times an L2, whose tiles are paced by what sets the call's time: every row against the float32
+    restatement, into a NaN-filled output."""
+    C = orc.cube_count(*grid)
+    video = C * 64 if layout == orc.CUBES_GATHERED else grid[0] * grid[1] * grid[2]
+    rows = video + n_dense
+    g = torch.Generator(device=dev).manual_seed(lists)
+    q, k, v = [torch.randn((heads, rows, 128), generator=g, device=dev).to(torch.bfloat16) for _ in range(3)]
+    idx = torch.rand((heads, C, C), generator=g, device=dev).topk(lists, 2).indices.int().sort(2).values.contiguous()
+    cnt = torch.full((heads, C), lists, dtype=torch.int32, device=dev)
+    a = mh.cube_args(heads, grid, layout=layout, head_stride=rows * 128, out_stride=lists)
+    for order in (None, mh.cube_order(a, idx, cnt)):
+        out = mh.flash_attn_sparse_128(a, q, k, v, idx, cnt, dense_row0=video, n_dense=n_dense,
+                                       out=nan_filled((heads, rows, 128), dev), order=order)
+        for h in range(heads):
+            ref = attn_sparse_f32(q, k, v, idx, cnt, grid, video, n_dense, layout=layout, heads=[h], chunk=32)
+            check_attn_f32(out, ref, f"{grid} head {h}")
+
+
+def test_flash_attn_sparse_dense_chain_keeps_its_pace(dev):
+    """A call of few heads and short lists takes as long as its dense tiles' chains over every key tile, and a key tile
+    of the chain takes as long in large heads (66 MB of K and V) as in smaller ones (38 MB): within 7%; it was 14%
+    slower where the large heads' dense tiles read their fragments at the cube tiles' pace."""
+    def per_key_tile(grid):
+        C = orc.cube_count(*grid)
+        video = grid[0] * grid[1] * grid[2]
+        q, k, v = [torch.randn((2, video + 64, 128), device=dev).to(torch.bfloat16) for _ in range(3)]
+        idx = torch.arange(C, dtype=torch.int32, device=dev).repeat(2, 1)[..., None].contiguous()
+        cnt = torch.ones((2, C), dtype=torch.int32, device=dev)
+        a = mh.cube_args(2, grid, head_stride=(video + 64) * 128, out_stride=1)
+        out = torch.empty_like(q)
+        return best_ms(lambda: mh.flash_attn_sparse_128(a, q, k, v, idx, cnt, dense_row0=video, n_dense=64,
+                                                        out=out)) / (C + 1)
+
+    large, small = per_key_tile((32, 48, 84)), per_key_tile((32, 48, 48))
+    assert large < 1.07 * small, f"{1e3 * large:.3f} us a key tile against {1e3 * small:.3f}"

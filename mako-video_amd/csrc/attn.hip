@@ -198,8 +198,8 @@ __device__ __forceinline__ bool tile_full(const Tile& r)
     return r.kind == 0 ? r.lim_t == 64u : (r.kind != 3 && r.lim_t == 4u && r.lim_y == 4u && r.lim_x == 4u);
 }
 
-// PACED: a call bound by the K/V stream past L2 (stream_bound), whose cube tiles read a fragment right before its MFMA;
-// the others read eight ahead.
+// PACED: a call of heads so large that its tiles may be bound by the K/V stream past L2 (stream_bound); those then read
+// a fragment right before its MFMA, all others eight ahead.
 template <bool PACK, bool PACED>
 __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams p)
 {
@@ -591,7 +591,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
         // walks (the lists' mean from 64 of the head's counts), by an eighth: at that share and below, both paces are
         // within 2% (5 heads of 2016 cubes, 512 dense rows: ratio 0.02 4.80 -> 4.22 ms, 0.05 5.35 -> 4.75, 0.1
         // 7.36 and 7.48; 1440 cubes at 0.1 3.87 -> 3.69, 1760 5.43 and 5.44).
-        bool eager = false;
+        bool eager = uint64_t(n_sel) * 5u >= p.cubes; // a list of a fifth of the cubes or more
         if (dense_q) {
             const int32_t n = p.cnt[uint64_t(h) * p.cubes + (uint64_t(lane) * p.cubes >> 6)];
             const float mean = wave_sum(float(min(max(n, 0), int32_t(p.out_stride)))) * (1.0f / 64.0f);
@@ -648,17 +648,15 @@ uint32_t share_of(uint32_t heads, uint64_t bytes)
     return share;
 }
 
-// Whether the call waits for the K/V stream past L2 rather than for its own work: a head's K and V (`bytes`) many times
-// an XCD's 4 MB of L2, and lists of so few of its cubes that the tiles on an XCD seldom want the same one at once. The
-// time is then the bytes past L2 over some 7.4 TB/s, whatever a tile's own work takes, and a steadier pace, which
-// keeps the tiles' sweeps together, beats a faster one: reading each fragment right before its MFMA, the hit rate is 41%
-// against 30% (2016 cubes, 40 heads, ratio 0.1: 348 and 418 GB past L2; 48.2 against 54.0 ms, overlapping lists 47.2 and
-// 52.0; 1440 cubes, independent lists 25.1 and 27.1). Elsewhere eight ahead are faster (2016 cubes, 8 heads, ratio 0.3:
-// 33.0 and 31.4 ms; 1024 cubes 12.9 and 12.6; 37 x 17 x 30 dense 16.3 and 15.5).
-bool stream_bound(uint64_t bytes, const mh3::AttnParams& p)
-{
-    return bytes > (40ull << 20) && uint64_t(p.out_stride) * 5u < p.cubes;
-}
+// Whether the call's cube tiles may wait for the K/V stream past L2 rather than for their own work: a head's K and V
+// (`bytes`) many times an XCD's 4 MB of L2. Where a list also holds so few of its cubes that the tiles on an XCD seldom
+// want the same one at once (a tile sees its own list's length; idx's width says nothing), the time is the bytes past L2
+// over some 7.4 TB/s, whatever a tile's own work takes, and a steadier pace, which keeps the tiles' sweeps together,
+// beats a faster one: reading each fragment right before its MFMA, the hit rate is 41% against 30% (2016 cubes, 40
+// heads, ratio 0.1: 348 and 418 GB past L2; 48.2 against 54.0 ms, overlapping lists 47.2 and 52.0; 1440 cubes,
+// independent lists 25.1 and 27.1). Elsewhere eight ahead are faster (2016 cubes, 8 heads, ratio 0.3: 33.0 and 31.4 ms;
+// 1024 cubes 12.9 and 12.6; 37 x 17 x 30 dense 16.3 and 15.5).
+bool stream_bound(uint64_t bytes) { return bytes > (40ull << 20); }
 
 // order: null for the plain entry point; `ordered`: the ordered one, which needs it.
 int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, const uint16_t* v, const int32_t* idx,
@@ -728,7 +726,7 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
     const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0;
     const auto kernel = pack                                                ? &attn_sparse_kernel<true, false>
-                        : stream_bound((video + args->n_dense) * 512ull, p) ? &attn_sparse_kernel<false, true>
+                        : stream_bound((video + args->n_dense) * 512ull) ? &attn_sparse_kernel<false, true>
                                                                             : &attn_sparse_kernel<false, false>;
     const void* kern = reinterpret_cast<const void*>(kernel);
     const size_t lds = kStageBytes + (pack ? kSegBytes : 0u);

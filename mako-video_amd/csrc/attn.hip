@@ -82,6 +82,7 @@ struct AttnParams {
     uint32_t share, groups, per, dense_per;
     uint32_t sweep; // cube workgroups an XCD runs at once (0: pass lists in plain order)
     uint32_t slots; // workgroups the chip runs at once
+    uint32_t eager_from; // list length from which a PACED call's cube tile reads eight ahead (eager_list)
     FastDiv div_plane, div_cw; // c / plane and c / cw by multiply-high: a key tile's cube coordinates cost a few
                                // scalar instructions instead of integer divisions
     float scale_log2;    // score scale times log2(e): softmax in base 2
@@ -588,16 +589,16 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
     } else {
         // A dense tile walks every key tile, and in a call of few heads that chain can take as long as all of the cube
         // tiles: it then reads eight ahead too. That is where it is longer than a workgroup's share of all the call's
-        // walks (the lists' mean from 64 of the head's counts), by an eighth: at that share and below, both paces are
-        // within 2% (5 heads of 2016 cubes, 512 dense rows: ratio 0.02 4.80 -> 4.22 ms, 0.05 5.35 -> 4.75, 0.1
-        // 7.36 and 7.48; 1440 cubes at 0.1 3.87 -> 3.69, 1760 5.43 and 5.44).
-        bool eager = uint64_t(n_sel) * 5u >= p.cubes; // a list of a fifth of the cubes or more
+        // walks (the lists' mean from 64 of the head's counts; 5 heads of 2016 cubes, 512 dense rows: ratio 0.02 4.80 ->
+        // 4.22 ms, 0.05 5.35 -> 4.75, 0.1 7.36 and 7.48; 1440 cubes at 0.1 3.87 -> 3.69, 1760 5.43 and 5.44), and where
+        // the cube tiles do (40 heads of 1440 with every cube selected: 224 ms all ahead, 247 but for the dense tiles).
+        bool eager = n_sel >= p.eager_from;
         if (dense_q) {
             const int32_t n = p.cnt[uint64_t(h) * p.cubes + (uint64_t(lane) * p.cubes >> 6)];
             const float mean = wave_sum(float(min(max(n, 0), int32_t(p.out_stride)))) * (1.0f / 64.0f);
             const float chain = float(p.cubes) + float(p.nd), dense = float(p.nd);
             const float walks = float(p.heads) * (float(p.cubes) * (mean + dense) + dense * chain);
-            eager = __builtin_amdgcn_readfirstlane(chain * float(p.slots) > 1.125f * walks);
+            eager = __builtin_amdgcn_readfirstlane(chain * float(p.slots) > walks || mean >= float(p.eager_from));
         }
         if (eager)
             run(Ahead8{});
@@ -649,14 +650,32 @@ uint32_t share_of(uint32_t heads, uint64_t bytes)
 }
 
 // Whether the call's cube tiles may wait for the K/V stream past L2 rather than for their own work: a head's K and V
-// (`bytes`) many times an XCD's 4 MB of L2. Where a list also holds so few of its cubes that the tiles on an XCD seldom
-// want the same one at once (a tile sees its own list's length; idx's width says nothing), the time is the bytes past L2
-// over some 7.4 TB/s, whatever a tile's own work takes, and a steadier pace, which keeps the tiles' sweeps together,
-// beats a faster one: reading each fragment right before its MFMA, the hit rate is 41% against 30% (2016 cubes, 40
-// heads, ratio 0.1: 348 and 418 GB past L2; 48.2 against 54.0 ms, overlapping lists 47.2 and 52.0; 1440 cubes,
-// independent lists 25.1 and 27.1). Elsewhere eight ahead are faster (2016 cubes, 8 heads, ratio 0.3: 33.0 and 31.4 ms;
-// 1024 cubes 12.9 and 12.6; 37 x 17 x 30 dense 16.3 and 15.5).
+// (`bytes`) many times an XCD's 4 MB of L2. The time is then the bytes past L2 over some 7.4 TB/s, whatever a tile's own
+// work takes, and a steadier pace, which keeps the tiles' sweeps together, beats a faster one: reading each fragment
+// right before its MFMA, the hit rate is 41% against 30% (2016 cubes, 40 heads, ratio 0.1: 348 and 418 GB past L2; 48.2
+// against 54.0 ms, overlapping lists 47.2 and 52.0; 1440 cubes, independent lists 25.1 and 27.1). In smaller heads eight
+// ahead are faster (1024 cubes 12.9 and 12.6; 37 x 17 x 30 dense 16.3 and 15.5).
 bool stream_bound(uint64_t bytes) { return bytes > (40ull << 20); }
+
+// Whether an XCD's resident cube workgroups (four a CU) are through the call's cube tiles in under 16 rounds.
+bool few_rounds(const mh3::AttnParams& p)
+{
+    return uint64_t(p.per) * ((p.heads + p.groups - 1u) / p.groups) < 8u * uint64_t(mh3::host::cu_count());
+}
+
+// The list length from which a tile of a stream-bound call reads eight ahead all the same (a tile sees its own list's
+// length; idx's width says nothing): every cube, which the tiles then walk together at either pace, unless the heads are
+// larger still and of whole cubes (40 heads of 2016 cubes: ratio 0.25 134 ms eight ahead and 119 paced, 0.3 177 and 140,
+// overlapping lists 170 and 138, 0.6 319 and 272, 1 495 and 460; 20 heads of 1440 at 0.3 37 and 36, 1 113 and 119; 40 of
+// 31 x 48 x 84 at 1 454 and 475). In a call of few rounds, of which the unrotated first ones are much, it is a fifth of
+// the cubes (8 heads of 2016: 0.3 31.0 and 31.9, 0.5 51.3 and 53.4), or a third where all XCDs share each head (5 heads
+// of 768 cubes: 0.2 1.85 and 1.77, 0.3 2.70 and 2.56).
+uint32_t eager_list(const mh3::AttnParams& p, uint64_t bytes, bool pack)
+{
+    if (few_rounds(p))
+        return p.share == 8u ? (p.cubes + 2u) / 3u : (p.cubes + 4u) / 5u;
+    return pack || bytes < (56ull << 20) ? p.cubes : ~0u;
+}
 
 // order: null for the plain entry point; `ordered`: the ordered one, which needs it.
 int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, const uint16_t* v, const int32_t* idx,
@@ -719,15 +738,17 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     p.div_plane = FastDiv::make(p.plane);
     p.div_cw = FastDiv::make(p.cw);
     p.nd = uint32_t(nd), p.layout = c.layout, p.out_stride = c.out_stride;
-    p.share = share_of(c.heads, (video + args->n_dense) * 512ull);
+    const uint64_t bytes = (video + args->n_dense) * 512ull; // a head's K and V
+    p.share = share_of(c.heads, bytes);
     p.groups = 8u / p.share, p.per = (p.cubes + p.share - 1u) / p.share, p.dense_per = (p.nd * p.heads + 7u) / 8u;
     const float scale = args->scale > 0.0f ? args->scale : 0.08838834764831845f; // 1 / sqrt(128)
     p.scale_log2 = scale * 1.4426950408889634f;
     const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
     const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0;
-    const auto kernel = pack                                                ? &attn_sparse_kernel<true, false>
-                        : stream_bound((video + args->n_dense) * 512ull) ? &attn_sparse_kernel<false, true>
-                                                                            : &attn_sparse_kernel<false, false>;
+    p.eager_from = eager_list(p, bytes, pack);
+    const auto kernel = pack                  ? &attn_sparse_kernel<true, false>
+                        : stream_bound(bytes) ? &attn_sparse_kernel<false, true>
+                                              : &attn_sparse_kernel<false, false>;
     const void* kern = reinterpret_cast<const void*>(kernel);
     const size_t lds = kStageBytes + (pack ? kSegBytes : 0u);
     if (const hipError_t e = host::allow_dynamic_lds(kern, lds); e != hipSuccess)

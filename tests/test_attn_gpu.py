@@ -406,6 +406,7 @@ def best_ms(call, runs=12):
 @pytest.mark.parametrize("heads,grid,layout,n_dense,lists", [
     (2, (32, 52, 52), orc.CUBES_GRID, 70, 27),        # 44 MB of K and V a head: the dense tiles' chains are the call
     (2, (32, 52, 52), orc.CUBES_GATHERED, 70, 500),   # and here the cube tiles are
+    (16, (32, 52, 52), orc.CUBES_GRID, 70, 500),      # many rounds of cube tiles an XCD
 ])
 def test_flash_attn_sparse_large_heads(dev, heads, grid, layout, n_dense, lists):
     """Heads of many times an L2, whose tiles are paced by what sets the call's time: every row against the float32
@@ -417,11 +418,12 @@ def test_flash_attn_sparse_large_heads(dev, heads, grid, layout, n_dense, lists)
     q, k, v = [torch.randn((heads, rows, 128), generator=g, device=dev).to(torch.bfloat16) for _ in range(3)]
     idx = torch.rand((heads, C, C), generator=g, device=dev).topk(lists, 2).indices.int().sort(2).values.contiguous()
     cnt = torch.full((heads, C), lists, dtype=torch.int32, device=dev)
+    cnt[:, ::3] = 9                                   # tiles of both paces side by side
     a = mh.cube_args(heads, grid, layout=layout, head_stride=rows * 128, out_stride=lists)
     for order in (None, mh.cube_order(a, idx, cnt)):
         out = mh.flash_attn_sparse_128(a, q, k, v, idx, cnt, dense_row0=video, n_dense=n_dense,
                                        out=nan_filled((heads, rows, 128), dev), order=order)
-        for h in range(heads):
+        for h in (0, heads - 1):
             ref = attn_sparse_f32(q, k, v, idx, cnt, grid, video, n_dense, layout=layout, heads=[h], chunk=32)
             check_attn_f32(out, ref, f"{grid} head {h}")
 

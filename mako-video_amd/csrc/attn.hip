@@ -654,7 +654,9 @@ uint32_t share_of(uint32_t heads, uint64_t bytes)
 // work takes, and a steadier pace, which keeps the tiles' sweeps together, beats a faster one: reading each fragment
 // right before its MFMA, the hit rate is 41% against 30% (2016 cubes, 40 heads, ratio 0.1: 348 and 418 GB past L2; 48.2
 // against 54.0 ms, overlapping lists 47.2 and 52.0; 1440 cubes, independent lists 25.1 and 27.1). In smaller heads eight
-// ahead are faster (1024 cubes 12.9 and 12.6; 37 x 17 x 30 dense 16.3 and 15.5).
+// ahead are faster (1024 cubes 12.9 and 12.6; 37 x 17 x 30 dense 16.3 and 15.5). Grids with cubes at their edges too: 5
+// heads of 31 x 48 x 84 7.42 and 7.10 ms, 32 x 45 x 80 5.78 and 5.62, 40 heads of 33 x 48 x 84 60.0 and 59.0, at ratio 0.3
+// 180 and 168.
 bool stream_bound(uint64_t bytes) { return bytes > (40ull << 20); }
 
 // Whether an XCD's resident cube workgroups (four a CU) are through the call's cube tiles in under 16 rounds.
@@ -744,11 +746,10 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     const float scale = args->scale > 0.0f ? args->scale : 0.08838834764831845f; // 1 / sqrt(128)
     p.scale_log2 = scale * 1.4426950408889634f;
     const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
-    const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0;
+    const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0, paced = stream_bound(bytes);
     p.eager_from = eager_list(p, bytes, pack);
-    const auto kernel = pack                  ? &attn_sparse_kernel<true, false>
-                        : stream_bound(bytes) ? &attn_sparse_kernel<false, true>
-                                              : &attn_sparse_kernel<false, false>;
+    const auto kernel = pack    ? paced ? &attn_sparse_kernel<true, true> : &attn_sparse_kernel<true, false>
+                        : paced ? &attn_sparse_kernel<false, true> : &attn_sparse_kernel<false, false>;
     const void* kern = reinterpret_cast<const void*>(kernel);
     const size_t lds = kStageBytes + (pack ? kSegBytes : 0u);
     if (const hipError_t e = host::allow_dynamic_lds(kern, lds); e != hipSuccess)

@@ -407,6 +407,8 @@ def best_ms(call, runs=12):
     (2, (32, 52, 52), orc.CUBES_GRID, 70, 27),        # 44 MB of K and V a head: the dense tiles' chains are the call
     (2, (32, 52, 52), orc.CUBES_GATHERED, 70, 500),   # and here the cube tiles are
     (16, (32, 52, 52), orc.CUBES_GRID, 70, 500),      # many rounds of cube tiles an XCD
+    (2, (31, 53, 53), orc.CUBES_GATHERED, 70, 27),    # the same with cubes at the grid's edges
+    (16, (31, 53, 53), orc.CUBES_GRID, 70, 600),      # and with rotated lists of more entries than a segment
 ])
 def test_flash_attn_sparse_large_heads(dev, heads, grid, layout, n_dense, lists):
     """Heads of many times an L2, whose tiles are paced by what sets the call's time: every row against the float32

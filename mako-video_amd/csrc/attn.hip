@@ -649,6 +649,12 @@ uint32_t share_of(uint32_t heads, uint64_t bytes)
     return share;
 }
 
+// Whether an XCD's resident cube workgroups (four a CU) are through the call's cube tiles in under 16 rounds.
+bool few_rounds(const mh3::AttnParams& p)
+{
+    return uint64_t(p.per) * ((p.heads + p.groups - 1u) / p.groups) < 8u * uint64_t(mh3::host::cu_count());
+}
+
 // Whether the call's cube tiles may wait for the K/V stream past L2 rather than for their own work: a head's K and V
 // (`bytes`) many times an XCD's 4 MB of L2. The time is then the bytes past L2 over some 7.4 TB/s, whatever a tile's own
 // work takes, and a steadier pace, which keeps the tiles' sweeps together, beats a faster one: reading each fragment
@@ -656,14 +662,9 @@ uint32_t share_of(uint32_t heads, uint64_t bytes)
 // against 54.0 ms, overlapping lists 47.2 and 52.0; 1440 cubes, independent lists 25.1 and 27.1). In smaller heads eight
 // ahead are faster (1024 cubes 12.9 and 12.6; 37 x 17 x 30 dense 16.3 and 15.5). Grids with cubes at their edges too: 5
 // heads of 31 x 48 x 84 7.42 and 7.10 ms, 32 x 45 x 80 5.78 and 5.62, 40 heads of 33 x 48 x 84 60.0 and 59.0, at ratio 0.3
-// 180 and 168.
-bool stream_bound(uint64_t bytes) { return bytes > (40ull << 20); }
-
-// Whether an XCD's resident cube workgroups (four a CU) are through the call's cube tiles in under 16 rounds.
-bool few_rounds(const mh3::AttnParams& p)
-{
-    return uint64_t(p.per) * ((p.heads + p.groups - 1u) / p.groups) < 8u * uint64_t(mh3::host::cu_count());
-}
+// 180 and 168. In calls of few rounds the line lies lower (5 heads, ratio 0.1: 768 cubes 1.52 and 1.44 ms, 1024 2.25 and
+// 2.11; 576 equal), 40 heads of 1024 cubes 12.6 and 12.9.
+bool stream_bound(uint64_t bytes, bool few) { return bytes > (uint64_t(few ? 20 : 40) << 20); }
 
 // The list length from which a tile of a stream-bound call reads eight ahead all the same (a tile sees its own list's
 // length; idx's width says nothing): every cube, which the tiles then walk together at either pace, unless the heads are
@@ -746,7 +747,7 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     const float scale = args->scale > 0.0f ? args->scale : 0.08838834764831845f; // 1 / sqrt(128)
     p.scale_log2 = scale * 1.4426950408889634f;
     const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
-    const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0, paced = stream_bound(bytes);
+    const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0, paced = stream_bound(bytes, few_rounds(p));
     p.eager_from = eager_list(p, bytes, pack);
     const auto kernel = pack    ? paced ? &attn_sparse_kernel<true, true> : &attn_sparse_kernel<true, false>
                         : paced ? &attn_sparse_kernel<false, true> : &attn_sparse_kernel<false, false>;
@@ -759,9 +760,12 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
         if (const hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kern, int(kAttnThreads), lds);
             e != hipSuccess)
             return host::hip_error(e);
-        // The sweep period: the cube workgroups an XCD holds at once (half or twice that measured slower).
+        // The sweep period: the cube workgroups an XCD holds at once (half or twice that measured slower), and a
+        // sixteenth more in stream-bound calls of few rounds, whose tiles then start a little behind those before them
+        // (5 heads of 2016 cubes: independent lists 7.35 -> 7.21 ms, overlapping 6.73 -> 6.56, ratio 0.15 10.9 -> 10.7;
+        // 40 heads 48.9 -> 50.3).
         p.slots = uint32_t(std::max(per_cu, 1)) * uint32_t(host::cu_count());
-        p.sweep = p.slots / 8u;
+        p.sweep = p.slots / 8u + (paced && few_rounds(p) ? p.slots / 128u : 0u);
     }
     hipLaunchKernelGGL(kernel, dim3(uint32_t(blocks)), dim3(kAttnThreads), lds, static_cast<hipStream_t>(stream), p);
     return host::check_launch();

@@ -742,11 +742,21 @@ int launch_attn(const MH3AttnArgs* args, const uint16_t* q, const uint16_t* k, c
     p.div_cw = FastDiv::make(p.cw);
     p.nd = uint32_t(nd), p.layout = c.layout, p.out_stride = c.out_stride;
     const uint64_t bytes = (video + args->n_dense) * 512ull; // a head's K and V
+    // Workgroups of a launch with `share` XCDs a head. A launch holds under 2^32 threads: shares that do not divide the
+    // cubes round up to up to 7 more workgroups a head, which millions of heads of one cube each do not have to spare.
+    const auto blocks_of = [&](uint32_t share) {
+        const uint64_t per = (cubes + share - 1u) / share, groups = 8u / share;
+        return 8u * ((nd * c.heads + 7u) / 8u + per * ((c.heads + groups - 1u) / groups));
+    };
     p.share = share_of(c.heads, bytes);
+    if (blocks_of(p.share) * kAttnThreads >= (1ull << 32))
+        p.share = 1u;
+    const uint64_t blocks = blocks_of(p.share);
+    if (blocks * kAttnThreads >= (1ull << 32))
+        return MH3_ERR_SHAPE;
     p.groups = 8u / p.share, p.per = (p.cubes + p.share - 1u) / p.share, p.dense_per = (p.nd * p.heads + 7u) / 8u;
     const float scale = args->scale > 0.0f ? args->scale : 0.08838834764831845f; // 1 / sqrt(128)
     p.scale_log2 = scale * 1.4426950408889634f;
-    const uint64_t blocks = 8ull * p.dense_per + 8ull * p.per * ((c.heads + p.groups - 1u) / p.groups);
     const bool pack = p.gt % 4u != 0 || p.gh % 4u != 0 || p.gw % 4u != 0, paced = stream_bound(bytes, few_rounds(p));
     p.eager_from = eager_list(p, bytes, pack);
     const auto kernel = pack    ? paced ? &attn_sparse_kernel<true, true> : &attn_sparse_kernel<true, false>

@@ -470,3 +470,15 @@ def test_flash_attn_sparse_wide_lists_cost_nothing(dev):
                                                            out=outs[-1]), runs=5))
     assert torch.equal(*outs)
     assert ms[1] < 1.06 * ms[0], f"{ms[1]:.2f} ms with wide lists against {ms[0]:.2f}"
+
+
+def test_flash_attn_sparse_millions_of_heads(dev):
+    """4,300,001 heads of one token (an odd count: eight XCDs share a head's one cube, seven of them idle) fit in a
+    launch: each output is its only key's value."""
+    heads = 4_300_001
+    q, k, v = [torch.randn((heads, 1, 128), device=dev, dtype=torch.bfloat16) for _ in range(3)]
+    idx = torch.zeros((heads, 1, 1), dtype=torch.int32, device=dev)
+    cnt = torch.ones((heads, 1), dtype=torch.int32, device=dev)
+    out = mh.flash_attn_sparse_128(mh.cube_args(heads, (1, 1, 1), head_stride=128, out_stride=1), q, k, v, idx, cnt,
+                                   out=nan_filled((heads, 1, 128), dev))
+    assert torch.equal(out, v)

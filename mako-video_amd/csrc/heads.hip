@@ -216,8 +216,10 @@ struct HeadsPoolParams {
     uint32_t parts; // workgroups a cube: workgroup i of them takes the head vectors 8 i .. + 7 of its rows
     uint32_t cube_wgs, wgs0, video0, video1; // workgroups of the cubes; then those of output rows [0, video0) (wgs0 of
                                              // them) and [video1, rows), the rows before and after the cubes'
+    uint32_t first; // the launch's first workgroup: a launch takes 2^22 of them
 };
 constexpr uint32_t kPoolThreads = 512;
+constexpr uint32_t kPoolLaunch = 1u << 22;           // workgroups a launch (2^31 threads)
 constexpr int kTabU = 6;                            // table values a thread has in flight (64 x 48 in one turn)
 constexpr int kPoolU = 4;                           // slots a group has in flight (8: equal, and spills)
 
@@ -227,14 +229,15 @@ heads_pool_kernel(HeadsPoolParams pp)
 {
     const HeadsParams& p = pp.hp;
     extern __shared__ float lds[];
-    if (blockIdx.x >= pp.cube_wgs) {
-        const uint32_t d = blockIdx.x - pp.cube_wgs, before = d < pp.wgs0;
+    const uint32_t wg = pp.first + blockIdx.x;
+    if (wg >= pp.cube_wgs) {
+        const uint32_t d = wg - pp.cube_wgs, before = d < pp.wgs0;
         const uint32_t r0 = before ? d * p.rows_per_block : pp.video1 + (d - pp.wgs0) * p.rows_per_block;
         heads_rows(p, r0, min(p.rows_per_block, (before ? pp.video0 : p.rows) - r0), lds);
         return;
     }
     const uint32_t tid = threadIdx.x, lane = tid & 63u, part = lane & 15u, grp = lane >> 4, wave = tid >> 6;
-    const uint32_t c = blockIdx.x / pp.parts, part_of = blockIdx.x - c * pp.parts;
+    const uint32_t c = wg / pp.parts, part_of = wg - c * pp.parts;
     const uint64_t orow0 = pp.row0 + uint64_t(c) * 64u;
     float* wt = lds;
     int32_t* srcs = reinterpret_cast<int32_t*>(lds + 256);
@@ -493,7 +496,13 @@ extern "C" int mh3_heads_partial_pool(const MH3HeadsArgs* args, const MH3CubeArg
     if (const hipError_t e = host::allow_dynamic_lds(reinterpret_cast<const void*>(&heads_pool_kernel), lds);
         e != hipSuccess)
         return host::hip_error(e);
-    hipLaunchKernelGGL(heads_pool_kernel, dim3(uint32_t(wgs)), dim3(kPoolThreads), lds,
-                       static_cast<hipStream_t>(stream), pp);
-    return host::check_launch();
+    // A launch holds under 2^32 threads, which the cubes alone stay below but their parts need not.
+    for (uint64_t first = 0; first < wgs; first += kPoolLaunch) {
+        pp.first = uint32_t(first);
+        hipLaunchKernelGGL(heads_pool_kernel, dim3(uint32_t(std::min<uint64_t>(wgs - first, kPoolLaunch))),
+                           dim3(kPoolThreads), lds, static_cast<hipStream_t>(stream), pp);
+        if (const int rc2 = host::check_launch(); rc2 != MH3_OK)
+            return rc2;
+    }
+    return MH3_OK;
 }

@@ -168,3 +168,25 @@ def test_heads_partial_pool_grid_layout_edges(dev, grid, heads, n_before, n_afte
                                 cube_layout=mh.CUBES_GRID, q=bufs[0], k=bufs[1], v=bufs[2] if with_v else None)
     for name, g, w in zip(("q", "k", "v", "qc", "kc"), got, want):
         assert same(g, w), name
+
+
+def test_heads_partial_pool_more_workgroups_than_a_launch(dev):
+    """4,194,305 cubes of 3 heads, two workgroups a cube: more than one launch's threads. Every output row written, and
+    the cubes at both ends and around the launches' border the same bits as calls of those cubes alone."""
+    heads, cubes, n = 3, 4_194_305, 64
+    rows = 4 * cubes
+    g = torch.Generator(device=dev).manual_seed(4)
+    x = torch.randn((rows // 5, 3 * heads * 128), generator=g, device=dev, dtype=torch.bfloat16).repeat(5, 1)
+    qkv = [torch.full((heads, rows, 128), 0x7FC0, dtype=torch.int16, device=dev).view(torch.bfloat16) for _ in "qkv"]
+    qc, kc = (torch.full((heads, cubes, 128), float("nan"), device=dev) for _ in "qk")
+    mh.heads_partial_pool(x, heads, (1, 1, rows), rot=0, layout="heads", cube_layout=mh.CUBES_GRID, q=qkv[0], k=qkv[1],
+                          v=qkv[2], qc=qc, kc=kc)
+    for t in (*qkv, qc, kc):
+        assert all(bool(torch.isfinite(h.amax()) & torch.isfinite(h.amin())) for h in t), "an output left unwritten"
+    border = (1 << 22) // 2                                          # cubes of the first launch
+    for c in (0, border - n // 2, cubes - n):
+        want = mh.heads_partial_pool(x[4 * c:4 * (c + n)], heads, (1, 1, 4 * n), rot=0, layout="heads",
+                                     cube_layout=mh.CUBES_GRID)
+        got = [t[:, 4 * c:4 * (c + n)] for t in qkv] + [t[:, c:c + n] for t in (qc, kc)]
+        for name, a, b in zip(("q", "k", "v", "qc", "kc"), got, want):
+            assert torch.equal(a, b), f"{name} at cube {c}"

@@ -501,6 +501,7 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
             lds_barrier(); // every wave is done with it before it is overwritten
         }
     };
+    // Every key tile of this workgroup's walk, at one pace.
     auto run = [&](auto ahead) {
         if constexpr (!PACK) {
             walk(
@@ -615,17 +616,15 @@ __global__ __launch_bounds__(kAttnThreads, 2) void attn_sparse_kernel(AttnParams
         for (int j = 0; j < 8; ++j)
             *reinterpret_cast<uint4*>(orow + 16 * j + 8u * hh) = uint4{0u, 0u, 0u, 0u};
     }
-    if (q_token || (!PACK && qtile.kind == 2)) {
+    if (q_token) {
         uint16_t* orow = p.out + hoff + qrow * p.row_stride;
 #pragma unroll
         for (int db = 0; db < 4; ++db)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const uint32_t d0 = 32u * db + 8u * g + 4u * hh;
-                const uint2 w = PACK || q_token ? uint2{pack_bf16(o[db][4 * g] * inv, o[db][4 * g + 1] * inv),
-                                                pack_bf16(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv)}
-                                        : uint2{0u, 0u}; // +0, not the sign of 0 * o
-                *reinterpret_cast<uint2*>(orow + d0) = w;
+                *reinterpret_cast<uint2*>(orow + d0) = uint2{pack_bf16(o[db][4 * g] * inv, o[db][4 * g + 1] * inv),
+                                                             pack_bf16(o[db][4 * g + 2] * inv, o[db][4 * g + 3] * inv)};
             }
     }
 }
@@ -637,10 +636,10 @@ namespace {
 
 // How many XCDs share one head's cube tiles (8, 4, 2 or 1), `bytes` being a head's K and V. Fewer XCDs a head mean more
 // of its query cubes on each L2 at once, over the same keys (56 heads, 33 x 15 x 35, 9 MB a head: 3.90 ms at 8, 3.72 at
-// 2 and 1; the dense 37 x 17 x 30: 23.2 and 22.5), but 8 / share heads' K and V in flight at once: past half of the
-// 256 MB MALL that begins to cost (40 heads of 66 MB, independent and overlapping lists: 53.0 and 49.4 ms at 8, 50.2
-// and 48.8 at 4, 49.0 and 50.2 at 2, 49.1 and 51.9 at 1). The heads must also divide over the groups (5 heads of 66 MB:
-// 6.7 ms at 8, 7.9 at 4, 9.4 at 1).
+// 2 and 1; the dense 37 x 17 x 30: 23.2 and 22.5), but 8 / share heads' K and V in flight at once, which costs as they
+// fill the 256 MB MALL (40 heads of 66 MB, independent and overlapping lists: 53.0 and 49.4 ms at 8, 50.2 and 48.8 at 4,
+// 49.0 and 50.2 at 2, 49.1 and 51.9 at 1). The limit of 144 MB lies just above two such heads, the most that was better
+// for both. The heads must also divide over the groups (5 heads of 66 MB: 6.7 ms at 8, 7.9 at 4, 9.4 at 1).
 uint32_t share_of(uint32_t heads, uint64_t bytes)
 {
     uint32_t share = 1;

@@ -1045,7 +1045,7 @@ int mh3_cube_select(const MH3CubeArgs* args, const float* qc, const float* kc, v
     hipLaunchKernelGGL(cube_split_kernel, dim3((blocks + 3u) / 4u), dim3(256), 0, st, g, kc, ks);
     if ((rc = host::check_launch()) != MH3_OK)
         return rc;
-    // Persistent: one workgroup a CU (the tile takes the LDS), at most one a tile.
+    // Persistent: one workgroup a CU (its 12 waves' registers, and at 32 cubes a lane the tile's LDS), at most one a tile.
     const uint32_t tiles = (g.cubes + kSelectRows - 1) / kSelectRows * g.heads;
     const dim3 grid(std::min<uint32_t>(tiles, uint32_t(host::cu_count())));
     hipLaunchKernelGGL(select, grid, dim3(kSelectThreads), lds, st, g, qc, kc, ks, args->k,

@@ -139,11 +139,11 @@ struct GemmGate {
 typedef int int32x4 __attribute__((ext_vector_type(4)));
 
 // The epilogue shared by the GEMM kernels, through the LDS (idle after the last K-step). acc[a][b][e] is y[r][c]
-// with c = lane % 16 + 16 b + wn 16 TN within the tile's first 128 w rows (b < TN) or, for acc[a][TN + b], the same
-// position in its second 128, and tile row r = wm (BM / WM) + a 16 + 4 (lane / 16) + e. A
-// 128-column half of the tile at a time, each wave writes its scaled results as floats into a [256][kEpiStride] LDS
+// with c = lane % 16 + 16 b + wn 16 TN within the tile's first BN w rows (b < TN) or, for acc[a][TN + b], the same
+// position in its second BN, and tile row r = wm (BM / WM) + a 16 + 4 (lane / 16) + e. A
+// BN-column half of the tile at a time, each wave writes its scaled results as floats into a [BM][kEpiStride] LDS
 // tile (the two half-waves' rows, 4 apart, fall on disjoint banks); then each thread takes 8 consecutive columns of
-// a row, so the output, and with kGateAdd the residual, moves in 16-byte accesses, 16 threads to a row's 256 bytes.
+// a row, so the output, and with kGateAdd the residual, moves in 16-byte accesses, BN / 8 threads to a row.
 // The results round to bf16 once, at the end, as they would written straight from the registers.
 template <int BM, int BN, int WM, int WN, int MODE, int EPI, int TM, int TN, typename Acc>
 __device__ __forceinline__ void gemm_epilogue(Acc (&acc)[TM][2 * TN], u32x4_t* smem, uint32_t M, uint32_t N,
@@ -252,15 +252,15 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
     uint32_t tm, tn;
     tile_of<BM>(mt, nt, tm, tn);
     const uint32_t m0 = tm * uint32_t(BM);
-    // The tile's two 128-row halves of w (and the output columns they give): gate and up rows, or consecutive rows.
+    // The tile's two BN-row halves of w (and the output columns they give): gate and up rows, or consecutive rows.
     const uint32_t w_lo = EPI == kSwiGLU ? tn * uint32_t(BN) : tn * 2u * BN;
     const uint32_t w_hi = EPI == kSwiGLU ? N + w_lo : w_lo + uint32_t(BN);
     const uint32_t w_rows = EPI == kSwiGLU ? 2u * N : N;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, wm = wave / WN, wn = wave % WN;
     const uint32_t KT = K / kKS;
 
-    // A: straight from global memory into the LDS ring (buffer_load ... lds). A stage is 2048 16-byte chunks; each
-    // wave fills 2048 / kWaves of them, 64 a instruction; lane L of instruction i lands in chunk q = (wave * AI + i) *
+    // A: straight from global memory into the LDS ring (buffer_load ... lds). A stage is kAChunks 16-byte chunks;
+    // each wave fills kAChunks / kWaves of them, 64 an instruction; lane L of instruction i lands in chunk q = (wave * AI + i) *
     // 64 + L = row * 8 + physical chunk and fetches the logical chunk the swizzle puts there. The descriptor starts
     // at this tile's first row; rows past M read zero.
     constexpr int AI = int(kAChunks / 64 / kWaves), BD = int(kBChunks / 64 / kWaves);
@@ -281,8 +281,8 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
             lds_dma16(ra, stage + i * 64, a_off[i], int(kt * 128u));
     };
 
-    // B: 16-byte int8 vectors into registers a K-step ahead, widened to bf16 into the B ring. The stage's 1024 int8
-    // chunks (256 B-rows x 4 k-chunks; rows 0..127 the gate rows n0.., 128..255 the up rows n + n0..) go BI to a
+    // B: 16-byte int8 vectors into registers kBRegs K-steps ahead, widened to bf16 into the B ring. The stage's 8 BN int8
+    // chunks (2 BN B-rows x 4 k-chunks; rows 0 .. BN - 1 the gate rows n0.., the others the up rows n + n0..) go BI to a
     // thread: chunk q = tid + kThreads i is k-chunk q % 4 of B-row 4 (G / 2) + 2 ((q / 4) % 2) + G % 2, G = q / 8.
     // Each 8 consecutive lanes thus write two rows whose swizzles differ in parity, i.e. 8 distinct chunk columns.
     constexpr int BI = int(BN * 8u / kThreads);
@@ -318,7 +318,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
             b_piece(kt, rb, p);
     };
     // bf16 weights, and int8 weights with int8 x: B goes straight into its LDS ring like A, B-row r of the tile from
-    // weight row n0 + r (gate) or n + n0 + r - 128 (up), with A's chunk-to-lane assignment and swizzle.
+    // weight row n0 + r (gate) or n + n0 + r - BN (up), with A's chunk-to-lane assignment and swizzle.
     uint32_t bd_off[BD];
 #pragma unroll
     for (int i = 0; i < BD && !I8; ++i) {
@@ -335,7 +335,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(
     };
 
     // MFMA operands, 16 bytes a lane (8 bf16 or 16 int8 of k). Sub-step ks: k-half h = ks/2 and the wave's row tiles
-    // (ks%2)*FA .. +FA-1, A rows wm*(256/WM) + t*16 + lane%16, B rows wn*16TN + t*16 + lane%16 (and 128 + that),
+    // (ks%2)*FA .. +FA-1, A rows wm*(BM/WM) + t*16 + lane%16, B rows wn*16TN + t*16 + lane%16 (and BN + that),
     // k-chunk 4h + lane/16. Every row a lane reads has (row >> 1) & 7 = (lane % 16 >> 1) & 7, so one offset per
     // sub-step serves all tiles; t moves it by 16 rows. (The 16 rows a quarter-wave reads at one chunk then cover the
     // 64 banks once.)

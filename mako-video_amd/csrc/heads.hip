@@ -16,7 +16,7 @@
 //   (the norm factor is the group's).
 // - The workgroup stages the two norm weight vectors and its rows' cos / sin tables in LDS once.
 // - A padding slot of the cube map writes zeros and reads nothing.
-// mh3_heads_partial_pool adds cube_pool to the same pass (heads_pool_kernel, a cube a workgroup): the selector's
+// mh3_heads_partial_pool adds cube_pool to the same pass (heads_pool_kernel, some workgroups a cube): the selector's
 // cube means come from the values as they are stored, so q and k are not read back from HBM.
 #include "mh3_common.hpp"
 
@@ -355,7 +355,7 @@ namespace {
 
 using namespace mh3;
 
-// The checks of mh3_heads_partial and the kernel parameters they give (row_begin 0, rows_per_block unset).
+// The checks of mh3_heads_partial and the kernel parameters they give.
 int heads_setup(const MH3HeadsArgs* args, const uint16_t* qkv, const float* q_w, const float* k_w,
                 const float* cos_t, const float* sin_t, const int32_t* map, uint16_t* q, uint16_t* k, uint16_t* v,
                 HeadsParams& p)
@@ -467,8 +467,8 @@ extern "C" int mh3_heads_partial_pool(const MH3HeadsArgs* args, const MH3CubeArg
     if (!host::aligned16(qc) || !host::aligned16(kc))
         return MH3_ERR_ALIGN;
     {
-        // The pooled outputs may not overlap any input, the head tiles this call writes, or each other: one
-        // workgroup a cube writes them while the others still read qkv and write their own rows.
+        // The pooled outputs may not overlap any input, the head tiles this call writes, or each other: a
+        // cube's workgroups write them while the others still read qkv and write their own rows.
         const uint64_t qkv_bytes = ((uint64_t(args->model_rows) - 1) * args->qkv_stride + 3ull * args->heads * 128u) * 2u;
         const uint64_t out_bytes = ((uint64_t(args->heads) - 1) * args->out_head_stride +
                                     (uint64_t(args->rows) - 1) * args->out_row_stride + 128u) * 2u;

@@ -50,7 +50,7 @@ CASES = [
     ((8, 8, 12), orc.CUBES_GRID, 5, 0, 0, 3, 0),
     ((4, 5, 4), orc.CUBES_GRID, 64, 0, 64, 1, 1),
     ((13, 10, 9), orc.CUBES_GRID, 0, 1170, 130, 6, 1),
-    # 64 cubes and 4 dense tiles x 2 heads, both multiples of 8: the XCD-sliced order with rotated pass lists
+    # 64 cubes in parts of 16, four XCDs a head
     ((16, 16, 16), orc.CUBES_GRID, 0, 4096, 256, 6, 1),
     ((15, 16, 16), orc.CUBES_GATHERED, 256, 0, 200, 9, 3),
 ]
@@ -305,7 +305,7 @@ def test_flash_attn_sparse_768p_40_heads(dev, ordered):
     print(f"768p 40 heads: worst element error {worst[0]:.3g}, worst row RMS error {worst[1]:.3g} of the row's RMS")
     nd = n_dense // 64
     rng = np.random.default_rng(16)
-    # cube c of head h lands in XCD slice c * 8 // C; cover every slice across the heads
+    # an eighth of the cubes each of eight heads in turn: every XCD's part of a head (a quarter, in raster order) twice
     tiles = [(h, int(rng.integers(0, nd))) for h in range(0, heads, 5)]
     tiles += [(h, nd + int(c)) for h in range(heads) for c in [((h % 8) * C) // 8 + int(rng.integers(0, C // 8))]]
     hs = sorted({h for h, _ in tiles})
@@ -482,3 +482,30 @@ def test_flash_attn_sparse_millions_of_heads(dev):
     out = mh.flash_attn_sparse_128(mh.cube_args(heads, (1, 1, 1), head_stride=128, out_stride=1), q, k, v, idx, cnt,
                                    out=nan_filled((heads, 1, 128), dev))
     assert torch.equal(out, v)
+
+
+@pytest.mark.parametrize("heads,grid,layout,n_dense,lists", [
+    (160, (15, 15, 15), orc.CUBES_GRID, 64, 9),        # 64 cubes, an XCD a head: ranks to 1279
+    (160, (15, 15, 15), orc.CUBES_GATHERED, 64, 9),
+    (24, (9, 42, 70), orc.CUBES_GRID, 40, 560),        # 594 cubes: ranks to 1781, lists of more than a segment
+])
+def test_flash_attn_sparse_packed_rotated_walk(dev, heads, grid, layout, n_dense, lists):
+    """Padded grids with enough cube tiles an XCD that most start a fraction of the way into their lists (rank 512 and
+    up at 4 workgroups a CU on 256 CUs), in the plain order and in cube_order's: every row of heads from the first,
+    unrotated rounds and of rotated ones against the float32 restatement, into a NaN-filled output."""
+    assert torch.cuda.get_device_properties(dev).multi_processor_count == 256
+    C = orc.cube_count(*grid)
+    video = C * 64 if layout == orc.CUBES_GATHERED else grid[0] * grid[1] * grid[2]
+    rows = video + n_dense
+    g = torch.Generator(device=dev).manual_seed(C + layout)
+    q, k, v = [torch.randn((heads, rows, 128), generator=g, device=dev).to(torch.bfloat16) for _ in range(3)]
+    idx = torch.rand((heads, C, C), generator=g, device=dev).topk(lists, 2).indices.int().sort(2).values.contiguous()
+    cnt = torch.full((heads, C), lists, dtype=torch.int32, device=dev)
+    cnt[:, 1::3] = lists - 5
+    a = mh.cube_args(heads, grid, layout=layout, head_stride=rows * 128, out_stride=lists)
+    for order in (None, mh.cube_order(a, idx, cnt)):
+        out = mh.flash_attn_sparse_128(a, q, k, v, idx, cnt, dense_row0=video, n_dense=n_dense,
+                                       out=nan_filled((heads, rows, 128), dev), order=order)
+        for h in (0, 1, heads // 2, heads - 9, heads - 1):
+            ref = attn_sparse_f32(q, k, v, idx, cnt, grid, video, n_dense, layout=layout, heads=[h], chunk=32)
+            check_attn_f32(out, ref, f"{grid} layout {layout} head {h}")

@@ -411,3 +411,23 @@ def test_cube_select_cubes_a_lane(dev, cubes):
             got = mh.cube_select(a, qc, kk)
             for x, y in zip(got, want):
                 assert torch.equal(x, y), f"{cubes} cubes, {name}, k {k}, local {local}"
+
+
+@pytest.mark.parametrize("grid", [(8, 4, 1020), (12, 4, 684), (8, 4, 1024), (12, 4, 1364), (8, 4, 2048), (12, 4, 1368)])
+def test_cube_select_neighbours_in_other_lanes(dev, grid):
+    """Two or three planes of cubes around the counts where a ranking lane holds 8, 16 or 32 of a row's cubes (510 to
+    1026): the neighbours in time that local 3 adds lie in other lanes. cube_select equal to cube_topk over cube_scores
+    and to the oracle, with more entries than local 1 gives."""
+    heads, cubes, k = 2, orc.cube_count(*grid), 7
+    g = torch.Generator(device=dev).manual_seed(cubes)
+    qc, kc = [torch.randn((heads, cubes, 128), generator=g, device=dev) for _ in range(2)]
+    a1, a3 = (mh.cube_args(heads, grid, k=k, local=local, out_stride=k + 3) for local in (1, 3))
+    s = mh.cube_scores(a3, qc, kc)
+    idx, cnt = mh.cube_select(a3, qc, kc)
+    for got, want in zip((idx, cnt), mh.cube_topk(a3, s)):
+        assert torch.equal(got, want)
+    widx, wcnt = orc.cube_topk(s.cpu().numpy().astype(np.float64), grid, k, 3, out_stride=k + 3,
+                              sorted_form=True)
+    assert (cnt.cpu().numpy() == wcnt).all() and (idx.cpu().numpy() == widx).all()
+    more = cnt - mh.cube_select(a1, qc, kc)[1]
+    assert bool((more >= 0).all()) and int(more.max()) >= len(range(0, grid[0], 4)) - 1

@@ -1,4 +1,7 @@
 """Parity of quant_rows_i8 (bit-exact) and the W8A16 fc1 GEMM + SwiGLU epilogue (bf16 at 1e-2) with the oracle."""
+import re
+from pathlib import Path
+
 import numpy as np
 import pytest
 import torch
@@ -227,12 +230,26 @@ def test_gemm_i8_768p_every_row(dev):
     assert_close(g, bits_to_f64(want), 1e-2, 1e-4, "int8 fc1 768p")
 
 
+def chosen_tile(m, nt, cus=256):
+    """The rows and columns of the tile that a launch of m rows and nt column tiles takes: the rule of choose_tile over
+    the table in the kernels' source."""
+    src = (Path(__file__).resolve().parent.parent / "mako-video_amd" / "csrc" / "gemm.hip").read_text()
+    table = re.search(r"kTiles\[\] = \{(.*?)\};", src)[1]
+    tiles = [tuple(map(int, t.split(","))) for t in re.findall(r"\{([^}]*)\}", table)]
+    return min(tiles, key=lambda t: -(-(-(-m // t[0]) * nt * (128 // t[1])) // cus) * t[2])[:2]
+
+
 @pytest.mark.parametrize("form", ["w8a16", "bf16", "w8a8"])
-@pytest.mark.parametrize("k", [128, 256, 384, 640])
+@pytest.mark.parametrize("k", [64, 128, 192, 256, 320, 384, 640])
 def test_gemm_row_tiles(dev, form, k):
     """Every tile (64 column tiles on 256 CUs: 1021 rows take 256-row tiles, 763 192, 505 128, 255 64, 33 the narrow
-    one), its last rows missing, at K-step counts around the LDS rings' depths: every element against float64 products, and the
+    one, by the launch's own table of costs), its last rows missing, at K-step counts around the LDS rings' depths: every element against float64 products, and the
     rows of a smaller batch bit-identical to the same rows of the larger one (the row tile changes no sum's order)."""
+    if form == "w8a8" and k % 128:
+        pytest.skip("W8A8 takes K in steps of 128")
+    assert torch.cuda.get_device_properties(dev).multi_processor_count == 256
+    assert [chosen_tile(m, 64) for m in (1021, 763, 505, 255, 33)] == [(256, 128), (192, 128), (128, 128), (64, 128),
+                                                                     (64, 32)]
     g = torch.Generator(device=dev).manual_seed(k)
     m_max, n = 1021, 64 * 128
     xf = torch.randn((m_max, k), generator=g, device=dev).to(torch.bfloat16)

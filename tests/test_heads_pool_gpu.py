@@ -155,7 +155,7 @@ def test_heads_partial_pool_grid_layout_768p(dev):
                                                                 ((5, 12, 20), 40, 0, 77, True), ((6, 4, 9), 3, 50, 0, False)])
 def test_heads_partial_pool_grid_layout_edges(dev, grid, heads, n_before, n_after, with_v):
     """The model's row order with frames of slots past the grid's edge, head vectors that do not fill the last
-    workgroup's 8 (21, 9, 6 of them a row), and rows before and after the grid's in the same launch: bit for bit the
+    workgroup's 8 (21 and 6 a row; 168 and 120 do fill it), and rows before and after the grid's in the same launch: bit for bit the
     two kernels, into outputs filled with NaN."""
     video = grid[0] * grid[1] * grid[2]
     rows = n_before + video + n_after

@@ -670,12 +670,15 @@ bool stream_bound(uint64_t bytes, bool few) { return bytes > (uint64_t(few ? 20 
 // larger still and of whole cubes (40 heads of 2016 cubes: ratio 0.25 134 ms eight ahead and 119 paced, 0.3 177 and 140,
 // overlapping lists 170 and 138, 0.6 319 and 272, 1 495 and 460; 20 heads of 1440 at 0.3 37 and 36, 1 113 and 119; 40 of
 // 31 x 48 x 84 at 1 454 and 475). In a call of few rounds, of which the unrotated first ones are much, it is a fifth of
-// the cubes (8 heads of 2016: 0.3 31.0 and 31.9, 0.5 51.3 and 53.4), or a third where all XCDs share each head (5 heads
-// of 768 cubes: 0.2 1.85 and 1.77, 0.3 2.70 and 2.56).
+// the cubes (8 heads of 2016: 0.3 31.0 and 31.9, 0.5 51.3 and 53.4), or, where all XCDs share each head, a third of the
+// key tiles, the dense ones among them (5 heads of 768 cubes: 0.2 1.85 and 1.77, 0.3 2.70 and 2.56; of 128 cubes and
+// 60,000 dense rows 14.2 and 14.5).
 uint32_t eager_list(const mh3::AttnParams& p, uint64_t bytes, bool pack)
 {
-    if (few_rounds(p))
-        return p.share == 8u ? (p.cubes + 2u) / 3u : (p.cubes + 4u) / 5u;
+    if (few_rounds(p)) {
+        const uint32_t third = (p.cubes + p.nd + 2u) / 3u;
+        return p.share == 8u ? third - std::min(third, p.nd) : (p.cubes + 4u) / 5u;
+    }
     return pack || bytes < (56ull << 20) ? p.cubes : ~0u;
 }
 

@@ -410,6 +410,7 @@ def best_ms(call, runs=12):
     (2, (31, 53, 53), orc.CUBES_GATHERED, 70, 27),    # the same with cubes at the grid's edges
     (16, (31, 53, 53), orc.CUBES_GRID, 70, 600),      # and with rotated lists of more entries than a segment
     (8, (24, 44, 44), orc.CUBES_GRID, 70, 60),        # 24 MB a head, few rounds, the last of them rotated
+    (5, (8, 32, 32), orc.CUBES_GRID, 35000, 13),      # most of its key tiles dense
 ])
 def test_flash_attn_sparse_large_heads(dev, heads, grid, layout, n_dense, lists):
     """Heads of many times an L2, whose tiles are paced by what sets the call's time: every row against the float32
